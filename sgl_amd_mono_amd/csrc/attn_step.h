@@ -26,10 +26,10 @@
 //          above the threshold and the lowest positions equal to it, ascending -> cache
 //          slots (page_table[p / 64] * 64 + p % 64) -> mailbox sel (glm53/check.py:100-117)
 //   split  (row, 64 selected tokens): sub-tiles of 64 tokens gathered from the FP8
-//          cache into LDS as they lie (q.k operands, widened exactly to bf16 in
-//          registers) and, their value dims, widened and transposed (p.v operands); q
-//          in registers; bf16 MFMA 16x16x32 for q.k (two waves a token tile, each half
-//          of the 576 dims) and p.v, the per-token scale folded into the logit and the
+//          cache into LDS as they lie, two buffers: q.k operands, and p.v operands by
+//          transposed LDS reads, both widened exactly to bf16 in registers; q in
+//          registers; bf16 MFMA 16x16x32 for q.k (two waves a token tile, each half of
+//          the 576 dims) and p.v, the per-token scale folded into the logit and the
 //          probability, online softmax -> the split's partials (bf16, 32 KB in one
 //          contiguous run) and (m, l), then its done word (mailbox sdone)
 //   merge  (row, head): once every split of the row is done,
@@ -64,7 +64,6 @@ constexpr int QK_STEPS = QK_HALF / 32;       // its bf16 MFMA k steps
 // dwords a cached FP8 row in LDS: 16-byte aligned, and 20 banks (mod 64) from the next
 // row, so the 16 rows of a q.k operand read fall on distinct banks
 constexpr int KF_W = DQK / 4 + 4;
-constexpr int VT_STRIDE = SUB + 8;           // bf16 a transposed value row (one dim) in LDS
 constexpr int PF_STRIDE = SUB + 4;           // f32 a logit row in LDS
 constexpr int PB_STRIDE = SUB + 8;           // bf16 a probability row in LDS
 constexpr int ROPE_CH = (DQK - DV) / 16;     // 16-byte chunks of a row past the value dims
@@ -102,14 +101,16 @@ struct TopkLds {
 // element type is split by the compiler into 4-byte pairs (the cast's alignment is
 // not known to it); through an array of the unit type it is one b128 / b64 access.
 struct SplitLds {
-  union {  // the sub-tile's cached rows as they lie (E4M3): q.k operands (8 dims a unit)
-    u32x4 kf16[SUB][KF_W / 4];
-    u32x2 kf8[SUB][KF_W / 2];
-  };
-  union {  // their first DV dims widened to bf16, a row a dim (vt_unit): p.v operands
-    u32x4 vt16[DV][VT_STRIDE / 8];  // 8 tokens a unit
-    u32x2 vt8[DV][VT_STRIDE / 4];   // 4 tokens a unit
-    u32x4 q16[NH][Q_UNITS];         // before the first sub-tile: the row's q (bf16)
+  // the cached rows of two sub-tiles as they lie (E4M3), sub-tile st in buffer st % 2:
+  // the q.k operands (8 dims a unit) and, read transposed, the p.v operands
+  union {
+    u32x4 kf16[2][SUB][KF_W / 4];
+    u32x2 kf8[2][SUB][KF_W / 2];
+    struct {
+      u32x4 first[SUB][KF_W / 4];  // kf16[0]
+      u32x4 q16[NH][Q_UNITS];      // until the second sub-tile's rows: the row's q (bf16)
+    };
+    u32x2 ot[2][SUB][KF_W / 2];  // after the last sub-tile: the partials, in the buffer it does not use
   };
   union {  // logits [dim half][head][token]: sums over dims [0, 288) and [288, 576)
     f32x4 pf4[2][NH][PF_STRIDE / 4];
@@ -124,12 +125,13 @@ struct SplitLds {
     i32x4 slot4[SPLIT_MAX / 4];
   };
   union {
-    float kvs[SUB];
-    f32x4 kvs4[SUB / 4];
+    float kvs[2][SUB];
+    f32x4 kvs4[2][SUB / 4];
   };
   float alpha[NH];
 };
-static_assert(KF_W % 4 == 0 && VT_STRIDE % 8 == 0 && PF_STRIDE % 4 == 0 && PB_STRIDE % 8 == 0, "16-byte units");
+static_assert(KF_W % 4 == 0 && PF_STRIDE % 4 == 0 && PB_STRIDE % 8 == 0, "16-byte units");
+static_assert(sizeof(SplitLds::q16) <= sizeof(SplitLds::first), "q inside the second sub-tile's buffer");
 static_assert(NH * 16 == AT && SUB == 16 * 4, "softmax: a 16-lane row a head, 4 tokens a lane");
 
 struct MergeLds {
@@ -200,6 +202,14 @@ MONO_DEV f32x4 mfma_fp4_opb(const u32x4& a, const u32x4& b, int sa, int sb) {
 template <bool HW>
 MONO_DEV uint32_t fp8x2_bf16(uint32_t w) {
   return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, HW));
+}
+
+// A 16-lane group's transposed read of 8 rows x 16 bytes of LDS: lane l gives the address
+// of bytes 8 (l % 2) .. of row l / 2 and gets byte l of each of the 8 rows.
+MONO_DEV u32x2 lds_tr8(const u32x2* p) {
+  typedef int32_t i32x2 __attribute__((ext_vector_type(2)));
+  typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2*)p));
 }
 
 // 8 E4M3 bytes (two dwords) -> 8 bf16: an MFMA operand of 8 consecutive k
@@ -867,49 +877,21 @@ class Step {
     }
   }
 
-  // The 16-byte unit of vt row d holding tokens 8 u .. 8 u + 7: a row's units XOR the
-  // row's 16-dim group, so the 32 dim groups a wave's transposed store spans fall on 8
-  // different bank groups instead of one (a p.v read stays one aligned unit).
-  MONO_DEV static int vt_unit(int d, int u) { return u ^ ((d >> 4) & 7); }
-
-  // Store sub-tile st's rows: as they lie into kf8, and the value dims widened to bf16
-  // and transposed into vt (a thread writes one dim of its 4 tokens as 8 bytes); the
-  // rows of empty slots as zeros.
-  // (the rows as they lie, for q.k; the thread's value chunks stay in w. `vt_now`: the
-  // transposed values now, else gather_store_vt later: a long split runs it under its q.k
-  // MFMAs, 0.4-0.9 us faster at 24 and 48 rows; one-sub-tile splits measured 0.3-0.6 us
-  // slower that way and transpose here)
-  MONO_DEV void gather_store(SplitLds& P, int st, const Gather& gt, u32x4 (&w)[4], bool vt_now) {
+  // Store sub-tile st's rows into its buffer as they lie, the rows of empty slots as
+  // zeros, and its scales. One copy serves q.k and p.v: a second, widened and transposed
+  // one (64 KB of LDS stores, 64 VALU a thread and two more barriers a sub-tile) put 0.7
+  // us on the chain of a one-sub-tile split (one row of 700 keys: 13.2 -> 12.5 us a launch).
+  MONO_DEV void gather_store(SplitLds& P, int st, const Gather& gt) {
     const int c = tid % (DV / 16), m = tid / (DV / 16);
     const int32_t* sl = P.slot + st * SUB;
+    u32x4(*kf)[KF_W / 4] = P.kf16[st % 2];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const bool live = sl[4 * m + k] >= 0;
-      w[k] = live ? gt.v[k] : u32x4{0u, 0u, 0u, 0u};
-      P.kf16[4 * m + k][c] = w[k];
-    }
-    if (vt_now) gather_store_vt(P, w);
+    for (int k = 0; k < 4; ++k) kf[4 * m + k][c] = sl[4 * m + k] >= 0 ? gt.v[k] : u32x4{0u, 0u, 0u, 0u};
     if (tid < ROPE_CH * SUB) {
       const int t = tid / ROPE_CH;
-      P.kf16[t][DV / 16 + tid % ROPE_CH] = sl[t] >= 0 ? gt.rope : u32x4{0u, 0u, 0u, 0u};
+      kf[t][DV / 16 + tid % ROPE_CH] = sl[t] >= 0 ? gt.rope : u32x4{0u, 0u, 0u, 0u};
     }
-    if (tid < SUB) P.kvs[tid] = sl[tid] >= 0 ? gt.sc : 0.f;
-  }
-
-  // The thread's value chunks widened to bf16 and transposed into vt.
-  MONO_DEV void gather_store_vt(SplitLds& P, const u32x4 (&w)[4]) {
-    const int c = tid % (DV / 16), m = tid / (DV / 16);
-#pragma unroll
-    for (int p = 0; p < 8; ++p) {  // dims 16 c + 2 p, 16 c + 2 p + 1
-      uint32_t b[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) b[k] = p % 2 ? fp8x2_bf16<true>(w[k][p / 2]) : fp8x2_bf16<false>(w[k][p / 2]);
-      const u32x2 lo = {__builtin_amdgcn_perm(b[1], b[0], 0x05040100u), __builtin_amdgcn_perm(b[3], b[2], 0x05040100u)};
-      const u32x2 hi = {__builtin_amdgcn_perm(b[1], b[0], 0x07060302u), __builtin_amdgcn_perm(b[3], b[2], 0x07060302u)};
-      const int h8 = 2 * vt_unit(16 * c, m / 2) + m % 2;
-      P.vt8[16 * c + 2 * p][h8] = lo;
-      P.vt8[16 * c + 2 * p + 1][h8] = hi;
-    }
+    if (tid < SUB) P.kvs[st % 2][tid] = sl[tid] >= 0 ? gt.sc : 0.f;
   }
 
   // Split j of row s's nsp: its selected tokens in sub-tiles of SUB, [32 j / nsp, 32 (j +
@@ -988,7 +970,9 @@ class Step {
 #pragma unroll
       for (int ks = 0; ks < QK_STEPS; ++ks)
         qa[a][ks] = __builtin_bit_cast(bf16x8, P.q16[16 * a + r][QK_HALF / 8 * (wave / 4) + 4 * ks + g]);
-    __syncthreads();  // every wave holds its q before the first sub-tile's rows overwrite it
+    gather_store(P, 0, gt);
+    __syncthreads();
+    if (LONG && nsub > 1) gather_load(P, 1, gt);
 
 #pragma unroll 1
     for (int st = 0; st < nsub; ++st) {
@@ -997,17 +981,12 @@ class Step {
       // and held across it
       const int lane = LONG ? opaque_v(tid) % WAVE : this->lane, g = lane / 16, r = lane % 16;
       const int wv = LONG ? opaque_v(tid) / WAVE : wave;
-      u32x4 w[4];
-      gather_store(P, st, gt, w, !LONG);
-      __syncthreads();
-      // the next sub-tile's rows, in flight while this one computes (in three parts, one
-      // before each phase)
-      const bool next = st + 1 < nsub;
-      if (next) gather_load_part(P, st + 1, gt, 0);
+      const int buf = LONG ? st % 2 : 0;
+      const bool next = LONG && st + 1 < nsub, next2 = LONG && st + 2 < nsub;
       // logits, transposed: A = 16 cached rows (FP8, widened in registers), B = 16 heads
       // of q; lane (g, r) ends with tokens 16 tt + 4 g + i of head 16 a + r
       {
-        const u32x2* krow = &P.kf8[16 * (wv % 4) + r][QK_HALF / 8 * (wv / 4) + g];
+        const u32x2* krow = &P.kf8[buf][16 * (wv % 4) + r][QK_HALF / 8 * (wv / 4) + g];
         u32x2 kw[QK_STEPS];
 #pragma unroll
         for (int ks = 0; ks < QK_STEPS; ++ks) kw[ks] = krow[4 * ks];
@@ -1021,14 +1000,12 @@ class Step {
         P.pf4[wv / 4][r][4 * (wv % 4) + g] = s0;
         P.pf4[wv / 4][16 + r][4 * (wv % 4) + g] = s1;
       }
-      if (LONG) gather_store_vt(P, w);  // under the q.k MFMAs (read by p.v, after the softmax's barrier)
-      if (next) gather_load_part(P, st + 1, gt, 1);
       __syncthreads();
       // online softmax: head tid / 16, tokens 4 (tid % 16) .. + 3; the head's reductions
       // inside the lane's 16-lane row (DPP)
       {
         const int ti = LONG ? opaque_v(tid) : tid, h = ti / 16, tq = ti % 16;
-        const f32x4 x0 = P.pf4[0][h][tq], x1 = P.pf4[1][h][tq], ks = P.kvs4[tq];
+        const f32x4 x0 = P.pf4[0][h][tq], x1 = P.pf4[1][h][tq], ks = P.kvs4[buf][tq];
         const i32x4 sl = P.slot4[st * (SUB / 4) + tq];
         float x[4];
 #pragma unroll
@@ -1046,10 +1023,17 @@ class Step {
         P.pb8[h][tq] = u32x2{pack_bf16x2(pr[0] * ks[0], pr[1] * ks[1]), pack_bf16x2(pr[2] * ks[2], pr[3] * ks[3])};
         if (tq == 0) P.alpha[h] = al;
       }
-      if (next) gather_load_part(P, st + 1, gt, 2);
+      // the next sub-tile's rows into the other buffer (its last readers, the p.v of the
+      // sub-tile before, are behind this phase's first barrier) and the rows after them
+      // on their way, in three parts, so no wave stalls in one issue burst
+      if (next) gather_store(P, st + 1, gt);
+      if (next2) gather_load_part(P, st + 2, gt, 0);
       __syncthreads();
-      // o^T[dims x heads] = alpha o^T + v^T p^T: A = 16 dims of the transposed values,
-      // B = 16 heads' probabilities, k = 32 tokens a step
+      if (next2) gather_load_part(P, st + 2, gt, 1);
+      // o^T[dims x heads] = alpha o^T + v^T p^T: A = 16 dims of the values, read transposed
+      // (a 16-lane group reads 8 tokens x 16 dims, two lanes a token, and each lane gets
+      // one dim of the 8 tokens) and widened, B = 16 heads' probabilities, k = 32 tokens
+      // a step
       {
         float alh[2];
 #pragma unroll
@@ -1066,17 +1050,17 @@ class Step {
 #pragma unroll
           for (int a = 0; a < 2; ++a) pv[a] = __builtin_bit_cast(bf16x8, P.pb16[16 * a + r][4 * kt + g]);
 #pragma unroll
-          for (int b = 0; b < 4; ++b) {
-            const int d = 64 * wv + 16 * b + r;
-            va[b] = __builtin_bit_cast(bf16x8, P.vt16[d][vt_unit(d, 4 * kt + g)]);
-          }
+          for (int b = 0; b < 4; ++b)
+            va[b] = fp8x8_bf16x8(lds_tr8(&P.kf8[buf][32 * kt + 8 * g + r / 2][8 * wv + 2 * b + r % 2]));
 #pragma unroll
           for (int b = 0; b < 4; ++b)
 #pragma unroll
             for (int a = 0; a < 2; ++a) acc[b][a] = mfma_bf16(va[b], pv[a], acc[b][a]);
         }
       }
-      __syncthreads();
+      if (next2) gather_load_part(P, st + 2, gt, 2);
+      // (no barrier: the next q.k reads the other buffer and writes the logits, read
+      // before this phase's barrier)
     }
     // the partials (bf16, the reference's split partials, kernel.py:4040-4066) staged as
     // [head][dim] in LDS (a lane's 4 consecutive dims of a head as 8 bytes), then stored
@@ -1085,8 +1069,9 @@ class Step {
     // (a head's row padded by 16 bytes: the 16 heads of a lane group's store fall on
     // distinct banks)
     constexpr int OT_ROW = DV / 8 + 1;  // 16-byte units a staged head row
-    u32x2* ot = &P.vt8[0][0];           // free after the last p.v step's barrier
-    static_assert(sizeof(P.vt8) >= NH * OT_ROW * 16, "partial staging");
+    // the buffer that the last sub-tile does not use (its readers are two barriers back)
+    u32x2* ot = &P.ot[LONG ? nsub % 2 : 1][0][0];
+    static_assert(sizeof(P.ot[0]) >= NH * OT_ROW * 16, "partial staging");
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
@@ -1098,7 +1083,7 @@ class Step {
     {
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
           A.mail.part + ((size_t)s * SPLITS + j) * NH * DV, 0, NH * DV * 2, BUF_DWORD3);
-      const u32x4* ot16 = &P.vt16[0][0];
+      const u32x4* ot16 = &P.kf16[LONG ? nsub % 2 : 1][0][0];
       constexpr int CH16 = NH * DV * 2 / 16;  // 16-byte chunks of the split's partials
 #pragma unroll
       for (int q = 0; q < CH16 / AT; ++q) {
