@@ -14,8 +14,11 @@
 //          plane the B operand of v_mfma_scale_f32_16x16x128_f8f6f4 with FP4 formats:
 //          the plane's E8M0 bytes are the MFMA's per-lane B scales as they lie (a
 //          lane's dword holds its key's scale for the page's four 16-key tiles).
-//          score = sum_h w_h relu(q_h . k) -> mailbox score, and the task's histogram
-//          of the keys' leading 8-bit digits -> mailbox hist1
+//          score = sum_h w_h relu(q_h . k) -> mailbox score, and the histogram of the
+//          keys' leading 8-bit digits -> mailbox rowh. Only rows of more than TOPK keys
+//          are scored (a shorter row selects every key). One chunk a workgroup where the
+//          grid holds a workgroup for every chunk of max_ctx; else each workgroup takes a
+//          contiguous run of the step's chunks (score_run)
 //   topk   (row, member of a team of 16): the row's scores as order-preserving u32
 //          keys, 2048 a member; an MSB-first 8-bit radix select of the 2048th largest
 //          key: digit 1 from the chunk histograms, digit 2 from the sum of the members'
@@ -53,6 +56,12 @@ constexpr int TMK = TEAM_LONG;  // members of a row's top-k team in this launch
 constexpr bool kLongSplits = false;
 constexpr int TMK = TEAM;
 #endif
+// the launch may run the front too (a whole layer): the attention waits for its outputs
+#ifdef MONO_ATTN_FRONT
+constexpr bool kFront = true;
+#else
+constexpr bool kFront = false;
+#endif
 
 constexpr int AT = 512;
 constexpr int AW = AT / WAVE;
@@ -81,8 +90,17 @@ enum { W_SCORE = 0, W_SEL = 1, W_PART = 2, W_TEAM = 3 };
 
 
 
+constexpr int RUN = 8;  // chunks of a score run held in LDS at a time (64 rows of 32 chunks: 8 a CU)
+static_assert(RUN <= AW, "a wave looks a chunk up");
+
 struct ScoreLds {
-  uint32_t hist[256];  // the task's leading-digit histogram
+  uint32_t hist[256];  // the leading-digit histogram of the row's chunks scored here
+  // a run's chunks: their page numbers, and the query (E2M1 rows, E8M0 scales, head
+  // weights) of the row that starts at, or runs into, chunk j
+  int32_t pg[RUN][CHUNK / PAGE];
+  u32x4 q[RUN][IH * ID / 32];
+  uint32_t qs[RUN][IH];
+  u32x2 qw[RUN][IH / 4];
 };
 
 struct TopkLds {
@@ -254,6 +272,8 @@ class Step {
   // (a row's merges_of(rows) merges of 32 / merges_of(rows) heads each cover its NH heads)
   MONO_DEV int n_tasks() const { return n_score() + A.rows * TMK + A.rows * (splits_of(A.rows) + merges_of(A.rows)); }
   MONO_DEV int n_topk() const { return A.rows * TMK; }
+  // after the scores: the list index at which the tasks after them are dealt
+  MONO_DEV int list_base() const { return base; }
 
   // This workgroup's tasks (false, workgroup-uniform: a wait failed).
   MONO_DEV bool tasks() {
@@ -264,17 +284,19 @@ class Step {
   // workgroup's top-k tasks and before its splits: the fused layer's deferred work.
   template <class Between>
   MONO_DEV bool tasks(Between&& between) {
-    const int n_sc = n_score(), n_topk = A.rows * TMK;
+    const int n_topk = A.rows * TMK;
     const int nsp = splits_of(A.rows);
     const int n_split = A.rows * nsp;
-    if (!score_stage(block_index(), A.rows * CH)) return false;
+    if (!scores()) return false;
     // a workgroup's list is ordered by stage: one loop a stage keeps each loop body to
-    // one task kind (and its registers)
-    int T = first_at_or_after(n_sc);
-    for (; T < n_sc + n_topk; T += G) {
+    // one task kind (and its registers). The list after the scores starts at `base` (a
+    // multiple of TMK); a task's timeline row is its list index + tl0.
+    const int tl0 = n_score() - base;
+    int T = first_at_or_after(base);
+    for (; T < base + n_topk; T += G) {
       const uint64_t t0 = now_ticks();
-      const bool ok = topk_member((T - n_sc) / TMK, (T - n_sc) % TMK);
-      stamp(T, t0, 1);
+      const bool ok = topk_member((T - base) / TMK, (T - base) % TMK);
+      stamp(T + tl0, t0, 1);
       if (!ok) return false;  // workgroup-uniform
     }
     if (!between()) return false;
@@ -282,28 +304,28 @@ class Step {
     // long splits above, in k_attn_long alone (MONO_ATTN_LONG): every other launch takes
     // at most LONG_ROWS rows.
     if (!kLongSplits || nsp == SPLITS) {
-      for (T = first_at_or_after(n_sc + n_topk); T < n_sc + n_topk + n_split; T += G) {
+      for (T = first_at_or_after(base + n_topk); T < base + n_topk + n_split; T += G) {
         const uint64_t t0 = now_ticks();
-        const int j = T - n_sc - n_topk;
+        const int j = T - base - n_topk;
         const bool ok = split_task<false>(j / SPLITS, j % SPLITS, SPLITS);
-        stamp(T, t0, 2);
+        stamp(T + tl0, t0, 2);
         if (!ok) return false;
       }
     } else {
-      for (T = first_at_or_after(n_sc + n_topk); T < n_sc + n_topk + n_split; T += G) {
+      for (T = first_at_or_after(base + n_topk); T < base + n_topk + n_split; T += G) {
         const uint64_t t0 = now_ticks();
-        const int j = T - n_sc - n_topk;
+        const int j = T - base - n_topk;
         const bool ok = split_task<true>(j / nsp, j % nsp, nsp);
-        stamp(T, t0, 2);
+        stamp(T + tl0, t0, 2);
         if (!ok) return false;
       }
     }
-    if (!kLongSplits || nsp == SPLITS) return merges<SPLITS, 1>(n_sc + n_topk + n_split);
+    if (!kLongSplits || nsp == SPLITS) return merges<SPLITS, 1>(base + n_topk + n_split);
 #ifdef MONO_ATTN_WIDE
-    return nsp == 8 ? merges<8, 4>(n_sc + n_topk + n_split) : merges<4, 8>(n_sc + n_topk + n_split);
+    return nsp == 8 ? merges<8, 4>(base + n_topk + n_split) : merges<4, 8>(base + n_topk + n_split);
 #else
-    if (nsp == 8) return merges<8, 4>(n_sc + n_topk + n_split);
-    return nsp == 5 ? merges<5, 8>(n_sc + n_topk + n_split) : merges<4, 8>(n_sc + n_topk + n_split);
+    if (nsp == 8) return merges<8, 4>(base + n_topk + n_split);
+    return nsp == 5 ? merges<5, 8>(base + n_topk + n_split) : merges<4, 8>(base + n_topk + n_split);
 #endif
   }
 
@@ -312,9 +334,12 @@ class Step {
   Lds& L;
   Guard gd;
   int tid, lane, wave, g, r, G, CH;
+  int base = 0;
   bool q_ready = false;  // the front's q has been awaited (a fused launch)
   uint64_t waited = 0;
 
+  // a row's chunks that are scored
+  MONO_DEV int live_chunks(int n) const { return n > TOPK || A.scores ? (n + CHUNK - 1) / CHUNK : 0; }
   MONO_DEV int row_len(int s) const { return min(max(A.seq_lens[s], 0), A.mail.max_ctx); }
   // row s's leading-digit histogram of the launch with this tag: launches alternate
   // between two copies, and each launch clears the copy its successor uses
@@ -347,201 +372,353 @@ class Step {
   MONO_DEV void mark_waited() { waited = now_ticks(); }
 
   // ---------------------------------------------------------------- score
-  // A score task's operands for one wave: the row's FP4 query (head tile ht = heads
-  // 16 ht ..), its head weights, and 128 keys = 2 pages = 8 tiles of 16 keys (lane
-  // (g, r) holds chunk g of key 16 t + r) with their pages' E8M0 dwords.
-  struct ScoreOps {
-    int s, c, k0, n;
+  // The row's FP4 query in a wave's MFMA operands (64 heads x 128 dims: head tile ht =
+  // heads 16 ht ..) with its scales and head weights.
+  struct Query {
     u32x4 qa[IH / 16];
     int qsc[IH / 16];
     uint32_t w2[IH / 16][2];
+  };
+  // A wave's 128 keys of a chunk = 2 pages = 8 tiles of 16 keys (lane (g, r) holds chunk
+  // g of key 16 t + r) with their pages' E8M0 dwords.
+  struct Keys {
     u32x4 kb[KTILES];
     uint32_t ks[KEYS_WAVE / PAGE];
-    int pg[KEYS_WAVE / PAGE];
   };
+  // The wave's two pages of a chunk as buffer resources: the page is the base, so a
+  // lane's offset is the same for every tile and chunk; with no records (past a run's
+  // last chunk) the loads return zeros without touching memory, and every turn issues
+  // the same loads.
+  struct Pages {
+    __amdgpu_buffer_rsrc_t kv[KEYS_WAVE / PAGE], sc[KEYS_WAVE / PAGE];
+  };
+  static constexpr int NT_LOAD = 2;  // buffer cache policy: nontemporal
 
-  MONO_DEV void score_load(int T, ScoreOps& o) {
-    score_where(T, o);
-    if (o.k0 >= o.n) return;
-    score_query(o);
-    score_keys(o);
+  // The lane's and the wave's indices afresh (from an opaque copy of the thread index), so
+  // a loop's addresses are derived inside it, not hoisted out of it and held across it.
+  struct Lane {
+    int lane, g, r, wave;
+  };
+  MONO_DEV Lane lane_now() const {
+    const unsigned t = (unsigned)opaque_v(tid);
+    __builtin_assume(t < AT);
+    return {(int)(t % WAVE), (int)(t % WAVE / 16), (int)(t % 16), __builtin_amdgcn_readfirstlane((int)(t / WAVE))};
   }
 
-  MONO_DEV void score_where(int T, ScoreOps& o) const {
-    o.s = T / CH;
-    o.c = T % CH;
-    o.k0 = o.c * CHUNK + wave * KEYS_WAVE;
-    o.n = row_len(o.s);
+  MONO_DEV Pages pages(const int (&pg)[KEYS_WAVE / PAGE], bool any) const {
+    Pages p;
+#pragma unroll
+    for (int i = 0; i < KEYS_WAVE / PAGE; ++i) {
+      const size_t u = (size_t)__builtin_amdgcn_readfirstlane(pg[i]);
+      p.kv[i] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(A.ikv) + u * (PAGE * ID / 2), 0,
+                                                  any ? PAGE * ID / 2 : 0, BUF_DWORD3);
+      p.sc[i] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(A.iks) + u * (PAGE * ID / 32), 0,
+                                                  any ? PAGE * ID / 32 : 0, BUF_DWORD3);
+    }
+    return p;
+  }
+  MONO_DEV static void key_tile(const Lane& z, Keys& k, const Pages& p, int kt) {
+    k.kb[kt] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(p.kv[kt / 4], z.g * (PAGE * 16) + z.r * 16,
+                                                                               (kt % 4) * 256, NT_LOAD));
+  }
+  MONO_DEV static void key_scales(const Lane& z, Keys& k, const Pages& p, int i) {
+    k.ks[i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_raw_buffer_load_b32(p.sc[i], z.g * PAGE + z.r * 4, 0, 0));
+  }
+  MONO_DEV static void key_load(const Lane& z, Keys& k, const Pages& p) {
+#pragma unroll
+    for (int kt = 0; kt < KTILES; ++kt) {  // issued in the order in which a run's turns issue and use them
+      key_tile(z, k, p, kt);
+      if (kt % 4 == 3) key_scales(z, k, p, kt / 4);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
 
-  MONO_DEV void score_query(ScoreOps& o) const {
-    if (o.k0 >= o.n) return;
+  MONO_DEV void query_load(int s, Query& o) const {
 #pragma unroll
     for (int ht = 0; ht < IH / 16; ++ht) {
-      const size_t row = (size_t)o.s * IH + 16 * ht + r;
+      const size_t row = (size_t)s * IH + 16 * ht + r;
       o.qa[ht] = ld_u32x4(A.iq + row * (ID / 2) + g * 16);
       o.qsc[ht] = A.iqs[row * (ID / 32) + g];
-      const u32x2 w4 = *reinterpret_cast<const u32x2*>(A.iw + (size_t)o.s * IH + 16 * ht + 4 * g);
+      const u32x2 w4 = *reinterpret_cast<const u32x2*>(A.iw + (size_t)s * IH + 16 * ht + 4 * g);
       o.w2[ht][0] = w4[0];
       o.w2[ht][1] = w4[1];
     }
   }
 
-  MONO_DEV void score_keys(ScoreOps& o) const {
-    if (o.k0 >= o.n) return;
-    int pg[KEYS_WAVE / PAGE];
-#pragma unroll
-    for (int i = 0; i < KEYS_WAVE / PAGE; ++i) pg[i] = page_of(o.s, o.k0 + i * PAGE);
-#pragma unroll
-    for (int kt = 0; kt < KTILES; ++kt)
-      o.kb[kt] = ld_nt_u32x4(A.ikv + ((size_t)(pg[kt / 4] * 4 + g) * PAGE + (kt % 4) * 16 + r) * 16);
-#pragma unroll
-    for (int i = 0; i < KEYS_WAVE / PAGE; ++i)
-      o.ks[i] = *reinterpret_cast<const uint32_t*>(A.iks + (size_t)(pg[i] * 4 + g) * PAGE + r * 4);
-  }
-
-  // The next task's query and page numbers; its key tiles and scales are issued from
-  // inside the current task's compute (score_compute), so no wave sits in one 70 KB
-  // issue burst (the CU's memory queue fills and stalls it) while it could compute.
-  MONO_DEV void score_load_head(int T, ScoreOps& o) const {
-    score_where(T, o);
-    if (o.k0 >= o.n) return;
-#pragma unroll
-    for (int i = 0; i < KEYS_WAVE / PAGE; ++i) o.pg[i] = page_of(o.s, o.k0 + i * PAGE);
-    score_query(o);  // after the page numbers: their wait does not wait for the query
-  }
-  MONO_DEV void score_key_tile(ScoreOps& o, int kt) const {
-    o.kb[kt] = ld_nt_u32x4(A.ikv + ((size_t)(o.pg[kt / 4] * 4 + g) * PAGE + (kt % 4) * 16 + r) * 16);
-  }
-  MONO_DEV void score_key_scales(ScoreOps& o) const {
-#pragma unroll
-    for (int i = 0; i < KEYS_WAVE / PAGE; ++i)
-      o.ks[i] = *reinterpret_cast<const uint32_t*>(A.iks + (size_t)(o.pg[i] * 4 + g) * PAGE + r * 4);
-  }
-
   // key tile kt's logits against the four head tiles of the query
-  MONO_DEV static void score_mfmas(const ScoreOps& o, int kt, f32x4 (&d)[IH / 16]) {
+  MONO_DEV static void score_mfmas(const Query& q, const Keys& k, int kt, f32x4 (&d)[IH / 16]) {
 #pragma unroll
     for (int ht = 0; ht < IH / 16; ++ht) {
       switch (kt % 4) {
-        case 0: d[ht] = mfma_fp4_opb<0>(o.qa[ht], o.kb[kt], o.qsc[ht], (int)o.ks[kt / 4]); break;
-        case 1: d[ht] = mfma_fp4_opb<1>(o.qa[ht], o.kb[kt], o.qsc[ht], (int)o.ks[kt / 4]); break;
-        case 2: d[ht] = mfma_fp4_opb<2>(o.qa[ht], o.kb[kt], o.qsc[ht], (int)o.ks[kt / 4]); break;
-        default: d[ht] = mfma_fp4_opb<3>(o.qa[ht], o.kb[kt], o.qsc[ht], (int)o.ks[kt / 4]); break;
+        case 0: d[ht] = mfma_fp4_opb<0>(q.qa[ht], k.kb[kt], q.qsc[ht], (int)k.ks[kt / 4]); break;
+        case 1: d[ht] = mfma_fp4_opb<1>(q.qa[ht], k.kb[kt], q.qsc[ht], (int)k.ks[kt / 4]); break;
+        case 2: d[ht] = mfma_fp4_opb<2>(q.qa[ht], k.kb[kt], q.qsc[ht], (int)k.ks[kt / 4]); break;
+        default: d[ht] = mfma_fp4_opb<3>(q.qa[ht], k.kb[kt], q.qsc[ht], (int)k.ks[kt / 4]); break;
       }
     }
   }
 
-  // The wave's 128 scores -> mailbox score (lane (g, r) ends with keys k0 + 16 g + r and
-  // k0 + 64 + 16 g + r, so each store covers 64 consecutive positions), then the task's
-  // histogram of their leading key digits, added into the row's histogram (the top-k's
-  // first radix pass) before the chunk is marked done (mailbox cdone). Every wave
-  // reaches the barriers; a wave past the row computes nothing.
-  MONO_DEV void score_compute(const ScoreOps& o, ScoreOps& nx, bool more) {
-    const bool live = o.k0 < o.n;  // wave-uniform
-    // the next task's key tiles: two an iteration over this task's tiles 2-5 (its page
-    // numbers, loaded first, have landed by then; tiles 4-7 measured 2.6 us slower at 48
-    // rows, their loads still in flight at the task's acknowledgement wait)
-    const bool nx_live = more && nx.k0 < nx.n;  // wave-uniform
-    float sc[2] = {0.f, 0.f};
-    if (live) {
-      float wv[IH / 16][4];
+  // The wave's 128 scores of a chunk: lane (g, r) ends with those of its keys 16 g + r and
+  // 64 + 16 g + r. NEXT: the keys of pages `np` are loaded into k, tile by tile, as this
+  // chunk's are consumed (they are used two chunks later: a run holds two chunks' keys).
+  template <bool NEXT>
+  MONO_DEV static void chunk_scores(const Lane& z, const Query& q, Keys& k, const Pages& np, float (&sc)[2]) {
+    float wv[IH / 16][4];
 #pragma unroll
-      for (int ht = 0; ht < IH / 16; ++ht) {
-        wv[ht][0] = bf16_lo(o.w2[ht][0]);
-        wv[ht][1] = bf16_hi(o.w2[ht][0]);
-        wv[ht][2] = bf16_lo(o.w2[ht][1]);
-        wv[ht][3] = bf16_hi(o.w2[ht][1]);
-      }
-      // a key tile's four head-tile MFMAs are issued together and the next tile's before
-      // this tile's results are consumed, so no MFMA's latency sits in front of its use
-      // (32 MFMAs a wave, each consumed at once, cost ~1 us of exposed latency)
-      f32x4 d[2][IH / 16];
-      score_mfmas(o, 0, d[0]);
-#pragma unroll
-      for (int kt = 0; kt < KTILES; ++kt) {
-        if (kt + 1 < KTILES) score_mfmas(o, kt + 1, d[(kt + 1) % 2]);
-        static_assert(KTILES % 2 == 0, "two tiles an iteration");
-        if (nx_live && kt >= 2 && kt < 2 + KTILES / 2) {
-          score_key_tile(nx, 2 * kt - 4);
-          score_key_tile(nx, 2 * kt - 3);
-        }
-        float part = 0.f;
-#pragma unroll
-        for (int ht = 0; ht < IH / 16; ++ht)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) part += wv[ht][i] * (d[kt % 2][ht][i] > 0.f ? d[kt % 2][ht][i] : 0.f);
-        part += __shfl_xor(part, 16, WAVE);  // every lane group now holds key 16 kt + r's sum
-        part += __shfl_xor(part, 32, WAVE);
-        if (kt % 4 == g) sc[kt / 4] = part;
-      }
-    } else if (nx_live) {
-#pragma unroll
-      for (int kt = 0; kt < KTILES; ++kt) score_key_tile(nx, kt);
+    for (int ht = 0; ht < IH / 16; ++ht) {
+      wv[ht][0] = bf16_lo(q.w2[ht][0]);
+      wv[ht][1] = bf16_hi(q.w2[ht][0]);
+      wv[ht][2] = bf16_lo(q.w2[ht][1]);
+      wv[ht][3] = bf16_hi(q.w2[ht][1]);
     }
-    if (nx_live) score_key_scales(nx);
-    bool kl[2];
+    // a key tile's four head-tile MFMAs are issued together and the next tile's before
+    // this tile's results are consumed, so no MFMA's latency sits in front of its use
+    // (32 MFMAs a wave, each consumed at once, cost ~1 us of exposed latency)
+    f32x4 d[2][IH / 16];
+    float part[KTILES];
+    score_mfmas(q, k, 0, d[0]);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int pos = o.k0 + 64 * i + 16 * g + r;
-      kl[i] = live && pos < o.n;
-      if (kl[i]) {
-        __hip_atomic_store(&A.mail.score[(size_t)o.s * A.mail.max_ctx + pos], __float_as_uint(sc[i]), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-        if (A.scores) A.scores[(size_t)o.s * A.mail.max_ctx + pos] = sc[i];
+    for (int kt = 0; kt < KTILES; ++kt) {
+      if (kt + 1 < KTILES) score_mfmas(q, k, kt + 1, d[(kt + 1) % 2]);
+      if (NEXT) {
+        __builtin_amdgcn_sched_barrier(0);  // the tile's registers are free from here on
+        key_tile(z, k, np, kt);
+        if (kt % 4 == 3) key_scales(z, k, np, kt / 4);
       }
+      part[kt] = 0.f;
+#pragma unroll
+      for (int ht = 0; ht < IH / 16; ++ht)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[kt] += wv[ht][i] * (d[kt % 2][ht][i] > 0.f ? d[kt % 2][ht][i] : 0.f);
+      asm volatile("" : "+v"(part[kt]));  // summed here: eight tiles' logits would not fit the registers
     }
+    // each key's sum over the four lane groups, (0 + 1) + (2 + 3): two tiles meet in a
+    // swap of 16-lane rows, two such pairs in a swap of halves, and tile 4 h + j's sums
+    // end in lane group j
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      sc[h] = swap_sum<32>(swap_sum<16>(part[4 * h], part[4 * h + 1]), swap_sum<16>(part[4 * h + 2], part[4 * h + 3]));
+  }
+  // 16: rows (a0 + a1, b0 + b1, a2 + a3, b2 + b3); 32: halves (a lo + a hi, b lo + b hi)
+  template <int LANES>
+  MONO_DEV static float swap_sum(float a, float b) {
+    const uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+    const auto v = LANES == 16 ? __builtin_amdgcn_permlane16_swap(x, y, false, false)
+                               : __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+  }
+
+  // The wave's scores of chunk c of row s (n keys) -> mailbox score (each store covers 64
+  // consecutive positions; the buffer drops those past the row) and the workgroup's
+  // leading-digit histogram.
+  MONO_DEV void chunk_store(const Lane& z, int s, int c, int n, const float (&sc)[2]) {
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(A.mail.score + (size_t)s * A.mail.max_ctx, 0, n * 4, BUF_DWORD3);
+    const int p0 = c * CHUNK + z.wave * KEYS_WAVE + z.lane;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(sc[i]), rs, (p0 + 64 * i) * 4, 0, SC1);
+    if (A.scores)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (p0 + 64 * i < n) A.scores[(size_t)s * A.mail.max_ctx + p0 + 64 * i] = sc[i];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) hist_add(L.u.sc.hist, p0 + 64 * i < n, radix_key(sc[i]) >> 24);
+  }
+
+  // Chunks c .. c + k - 1 of row s are scored here: their histogram is added into the row's
+  // (the top-k's first radix pass) and, once every score and count is performed, they are
+  // marked done (mailbox cdone). Frees the histogram for the next row.
+  MONO_DEV void row_flush(int s, int c, int k) {
     uint32_t* hist = L.u.sc.hist;
-    __syncthreads();  // the previous task's histogram is added and cleared
-#pragma unroll
-    for (int i = 0; i < 2; ++i) hist_add(hist, kl[i], radix_key(sc[i]) >> 24);
     __syncthreads();
-    if (o.c * CHUNK < o.n) {  // workgroup-uniform
-      uint32_t* rh = row_hist(gd.tag, o.s);
-      if (tid < 256 && hist[tid] != 0u)
-        __hip_atomic_fetch_add(&rh[tid], hist[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __builtin_amdgcn_s_waitcnt(0);  // every add is performed before the chunk is marked done
-      __syncthreads();
-      if (tid == 0) mb_put(&A.mail.cdone[(size_t)o.s * CH + o.c], 0u, gd.tag);
-    }
+    uint32_t* rh = row_hist(gd.tag, s);
+    if (tid < 256 && hist[tid] != 0u)
+      __hip_atomic_fetch_add(&rh[tid], hist[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (tid < 256) hist[tid] = 0u;
+    __builtin_amdgcn_s_waitcnt(0);  // every score is stored and every add performed
+    __syncthreads();
+    if (tid < k) mb_put(&A.mail.cdone[(size_t)s * CH + c + tid], 0u, gd.tag);
   }
 
-  // The workgroup's score tasks T0, T0 + G, ... < n_score, each task's loads issued
-  // before the previous task computes.
-  MONO_DEV bool score_stage(int T0, int n_score) {
-    if (T0 >= n_score) return true;
-    if (tid < 256) L.u.sc.hist[tid] = 0u;
-    ScoreOps cur, nxt;
-    if (A.fdone) {
-      // the front of this launch writes each row's index query, head weights and new
-      // key: the first task's keys stream before the wait, except a wave's whose 128
-      // keys may hold a key written in this launch (the row's last `rows` positions: its
-      // own new key and, for the rows of a verify chain, those of the chain's earlier
-      // rows), then every row's front outputs are awaited
-      score_where(T0, cur);
-      const bool fresh = cur.k0 < cur.n && cur.k0 + KEYS_WAVE > cur.n - A.rows;  // wave-uniform
-      if (!fresh) score_keys(cur);
-      const uint64_t* fd = done_copy(A.fdone);
-      const int nr = A.rows;
-      if (!hint_wait(nr * (1 + IH / 8), [fd, nr](int i) { return fd + (i < nr ? proj::FD_B + i : proj::FD_E + i - nr); },
-                     A.fsite, gd))
-        return false;
-      if (fresh) score_keys(cur);
-      score_query(cur);
+  // In a launch that runs the front too, it writes each row's index query, head weights
+  // and new key: keys may be read before the wait for it (await_front), except a wave's
+  // whose pages may hold a key written in this launch (the row's last `rows` positions: its
+  // own new key and, for the rows of a verify chain, those of the chain's earlier rows;
+  // a wave past the row reads the row's last page).
+  MONO_DEV bool fresh(int k0, int n) const { return front_here() && k0 + KEYS_WAVE > n - A.rows; }  // wave-uniform
+  MONO_DEV bool front_here() const { return kFront && A.fdone; }
+  MONO_DEV bool await_front() {
+    const uint64_t* fd = done_copy(A.fdone);
+    const int nr = A.rows;
+    return hint_wait(nr * (1 + IH / 8), [fd, nr](int i) { return fd + (i < nr ? proj::FD_B + i : proj::FD_E + i - nr); },
+                     A.fsite, gd);
+  }
+
+  // This workgroup's share of the scores, and `base` for the tasks after them.
+  MONO_DEV bool scores() {
+    if (A.rows * CH > G) {
+      if (!score_run()) return false;
     } else {
-      score_load(T0, cur);
-    }
-    for (int T = T0; T < n_score; T += G) {
-      const uint64_t t0 = now_ticks();
-      const bool more = T + G < n_score;
-      if (more) score_load_head(T + G, nxt);
-      score_compute(cur, nxt, more);
-      stamp(T, t0, 0);
-      if (more) cur = nxt;
+      // a workgroup for every chunk of max_ctx: chunk b, with no look at the other rows'
+      // lengths in front of its loads (a round trip, ~1 us at 8 rows)
+      base = n_score();
+      const int b = block_index();
+      if (b < A.rows * CH) {
+        const int s = b / CH, c = b % CH, n = row_len(s);
+        if (c < live_chunks(n) && !score_one(s, c, n)) return false;  // workgroup-uniform
+      }
     }
     __syncthreads();  // the top-k tasks reuse the LDS
     return true;
+  }
+
+  MONO_DEV bool score_one(int s, int c, int n) {
+    const uint64_t t0 = now_ticks();
+    const Lane z = lane_now();
+    if (tid < 256) L.u.sc.hist[tid] = 0u;
+    const int k0 = c * CHUNK + z.wave * KEYS_WAVE;
+    int pg[KEYS_WAVE / PAGE];
+#pragma unroll
+    for (int i = 0; i < KEYS_WAVE / PAGE; ++i) pg[i] = page_of(s, min(k0 + i * PAGE, n - 1));
+    Query q;
+    Keys k;
+    if (!front_here()) query_load(s, q);
+    const Pages p = pages(pg, true);
+    const bool fr = fresh(k0, n);
+    if (!fr) key_load(z, k, p);
+    if (front_here()) {
+      if (!await_front()) return false;
+      if (fr) key_load(z, k, p);
+      query_load(s, q);
+    } else {
+      __syncthreads();  // the histogram is cleared
+    }
+    float sc[2];
+    chunk_scores<false>(z, q, k, p, sc);
+    chunk_store(z, s, c, n, sc);
+    row_flush(s, c, 1);
+    stamp(s * CH + c, t0, 0);
+    return true;
+  }
+
+  // The step's scored chunks, row by row, in contiguous runs of equal length (a chunk a
+  // workgroup while they last): every CU streams the same share whatever the rows'
+  // lengths, and a run pays the histogram's flush, its acknowledgement and the query once
+  // a row. Each chunk's keys are loaded two chunks ahead, so 64 to 128 KB a CU stay in
+  // flight and no wait drains them but a row's flush. Chunks dealt round-robin over
+  // max_ctx left three quarters of the grid idle at 33 rows of 1500-12000 keys (scores
+  // done after 22.4 us, now 6.0; the launch 63.6 -> 51.6), and each chunk's own flush
+  // drained its successor's loads (48 rows of 32768: 31.2 us, 3.4 TB/s, now 23.9, 4.5;
+  // the launch 76.0 -> 70.5).
+  MONO_DEV bool score_run() {
+    ScoreLds& P = L.u.sc;
+    const int nl = lane < A.rows ? row_len(lane) : 0;
+    const int inc = wave_incl_scan(live_chunks(nl));
+    const int total = __builtin_amdgcn_readlane(inc, WAVE - 1), b = block_index();
+    base = (min(total, G) + TMK - 1) / TMK * TMK;
+    int i0 = total > G ? (int)((int64_t)b * total / G) : min(b, total);
+    const int i1 = total > G ? (int)((int64_t)(b + 1) * total / G) : min(b + 1, total);
+    if (i0 >= i1) return true;  // workgroup-uniform
+    if (tid < 256) P.hist[tid] = 0u;
+    // row s of scored chunk i, and the row's first one
+    const auto row_at = [inc](int i) { return (int)__popcll(__ballot(inc <= i)); };
+    const auto first_of = [inc](int s) { return s > 0 ? __builtin_amdgcn_readlane(inc, s - 1) : 0; };
+    bool awaited = !front_here();
+#pragma unroll 1
+    for (; i0 < i1; i0 += RUN) {
+      const Lane z = lane_now();
+      const int m = min(i1 - i0, RUN);  // chunks of this piece
+      __syncthreads();  // the piece before is done with the LDS; the histogram is cleared
+      bool lead = false;
+      int s = 0;
+      if (z.wave < m) {  // wave w looks up chunk w
+        s = row_at(i0 + z.wave);
+        const int f = first_of(s), n = __builtin_amdgcn_readlane(nl, s);
+        const int p0 = (i0 + z.wave - f) * CHUNK + (z.lane % (CHUNK / PAGE)) * PAGE;
+        const int pg = page_of(s, min(p0, n - 1));
+        lead = z.wave == 0 || f == i0 + z.wave;  // wave-uniform: the row's first chunk of the piece
+        if (awaited && lead) run_query(z, s);
+        if (z.lane < CHUNK / PAGE) P.pg[z.wave][z.lane] = pg;
+      }
+      __syncthreads();
+      const auto pages_of = [&](const Lane& z, int j) {
+        int pg[KEYS_WAVE / PAGE];
+#pragma unroll
+        for (int i = 0; i < KEYS_WAVE / PAGE; ++i) pg[i] = P.pg[min(j, m - 1)][z.wave * (KEYS_WAVE / PAGE) + i];
+        return pages(pg, j < m);
+      };
+      Keys ka, kb;
+      if (awaited) {
+        key_load(z, ka, pages_of(z, 0));
+        key_load(z, kb, pages_of(z, 1));
+      } else {
+        const auto fresh_at = [&](int j) {
+          const int sj = row_at(i0 + min(j, m - 1));
+          return fresh((i0 + j - first_of(sj)) * CHUNK + z.wave * KEYS_WAVE, __builtin_amdgcn_readlane(nl, sj));
+        };
+        const bool fa = fresh_at(0), fb = fresh_at(1);
+        if (!fa) key_load(z, ka, pages_of(z, 0));
+        if (!fb) key_load(z, kb, pages_of(z, 1));
+        if (!await_front()) return false;
+        awaited = true;
+        if (lead) run_query(z, s);
+        if (fa) key_load(z, ka, pages_of(z, 0));
+        if (fb) key_load(z, kb, pages_of(z, 1));
+        __syncthreads();
+      }
+      Query q;
+      int n = 0, c = -1, c0 = 0;
+      const auto turn = [&](Keys& k, int j) {  // chunk j of the piece
+        const uint64_t t0 = now_ticks();
+        const Lane z = lane_now();
+        if (c < 0) {  // the row's first chunk of the piece
+          s = row_at(i0 + j);
+          n = __builtin_amdgcn_readlane(nl, s);
+          c = c0 = i0 + j - first_of(s);
+          query_from(z, j, q);
+        }
+        float sc[2];
+        chunk_scores<true>(z, q, k, pages_of(z, j + 2), sc);
+        chunk_store(z, s, c, n, sc);
+        const bool last = j + 1 == m || (c + 1) * CHUNK >= n;
+        if (last) row_flush(s, c0, c + 1 - c0);
+        stamp(s * CH + c, t0, 0);
+        c = last ? -1 : c + 1;
+      };
+#pragma unroll 1
+      for (int j = 0; j < m; j += 2) {
+        turn(ka, j);
+        if (j + 1 == m) break;
+        turn(kb, j + 1);
+      }
+    }
+    return true;
+  }
+  // Row s's query into the wave's LDS slot, and from slot j into a wave's operands.
+  MONO_DEV void run_query(const Lane& z, int s) {
+    ScoreLds& P = L.u.sc;
+    constexpr int N = IH * ID / 32 / WAVE;
+    u32x4 v[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = ld_u32x4(A.iq + (size_t)s * (IH * ID / 2) + (WAVE * i + z.lane) * 16);
+    const uint32_t qs = *reinterpret_cast<const uint32_t*>(A.iqs + ((size_t)s * IH + z.lane) * (ID / 32));
+    const u32x2 w = *reinterpret_cast<const u32x2*>(A.iw + (size_t)s * IH + z.lane % (IH / 4) * 4);
+#pragma unroll
+    for (int i = 0; i < N; ++i) P.q[z.wave][WAVE * i + z.lane] = v[i];
+    P.qs[z.wave][z.lane] = qs;
+    if (z.lane < IH / 4) P.qw[z.wave][z.lane] = w;
+  }
+  MONO_DEV void query_from(const Lane& z, int j, Query& o) const {
+    const ScoreLds& P = L.u.sc;
+#pragma unroll
+    for (int ht = 0; ht < IH / 16; ++ht) {
+      o.qa[ht] = P.q[j][(16 * ht + z.r) * (ID / 32) + z.g];
+      o.qsc[ht] = (int)((P.qs[j][16 * ht + z.r] >> (8 * z.g)) & 0xffu);
+      const u32x2 w4 = P.qw[j][4 * ht + z.g];
+      o.w2[ht][0] = w4[0];
+      o.w2[ht][1] = w4[1];
+    }
   }
 
   // ---------------------------------------------------------------- top-k
@@ -919,7 +1096,7 @@ class Step {
       split_done(s, j);
       return true;
     }
-    if (A.fdone && !q_ready) {  // every head of q from the front of this launch
+    if (front_here() && !q_ready) {  // every head of q from the front of this launch
       const uint64_t* fd = done_copy(A.fdone) + proj::FD_D;
       if (!hint_wait(NH, [fd](int i) { return fd + i; }, A.fsite + 1, gd)) return false;
       q_ready = true;
@@ -1117,7 +1294,7 @@ class Step {
       const uint64_t t0 = now_ticks();
       const int k = T - at;
       const bool ok = merge_task<NSP, HM>(k / MPR, k % MPR);
-      stamp(T, t0, 3);
+      stamp(T + n_score() - base, t0, 3);
       if (!ok) return false;
     }
     return true;

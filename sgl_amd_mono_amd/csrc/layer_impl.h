@@ -3,6 +3,7 @@
 // arguments, the LDS union and the phase sequence of one layer.
 #pragma once
 
+#define MONO_ATTN_FRONT 1
 #include "attn_step.h"
 #include "back_impl.h"
 #include "front_impl.h"
@@ -85,9 +86,8 @@ MONO_DEV bool run_layer(const LayerArgs& args, LayerLds& lds, const Guard& g, bo
   st.adopt(g);
   // Stage D (the absorbed query, read only by the splits) leaves the front when the
   // workgroups after the top-k teams can take it: head d runs on workgroup
-  // (scores + top-k tasks + d) mod G between its score and split tasks, which holds no
+  // (list base + top-k tasks + d) mod G between its score and split tasks, which holds no
   // top-k task, so no score task waits behind a D task.
-  const int d0 = st.n_score() + st.n_topk();
   const bool defer_d = st.n_topk() + proj::HEADS <= (int)gridDim.x;
   {
     proj::fr::Front f(args.fr, lds.fr);
@@ -99,7 +99,7 @@ MONO_DEV bool run_layer(const LayerArgs& args, LayerLds& lds, const Guard& g, bo
   __syncthreads();  // the LDS passes from the front's layout to the attention's
   const auto deferred = [&]() -> bool {
     if (!defer_d) return true;
-    const int G = (int)gridDim.x, b = (int)block_index();
+    const int G = (int)gridDim.x, b = (int)block_index(), d0 = st.list_base() + st.n_topk();
     for (int d = ((b - d0) % G + G) % G; d < proj::HEADS; d += G) {
       __syncthreads();  // the LDS passes to the front's layout
       proj::fr::Front f(args.fr, lds.fr);

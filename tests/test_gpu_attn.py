@@ -125,6 +125,33 @@ def test_attn_56_rows_wide_launch(rt, gpu_device):
     _check(rt, ctx, 13, gpu_device)
 
 
+@pytest.mark.parametrize("rows", [9, 13, 33, 64])
+def test_attn_score_runs(rt, gpu_device, rows):
+    """More rows than the grid has a workgroup for every chunk: the scored chunks run in
+    contiguous shares over the workgroups. Rows around the selection's and the chunks'
+    edges against the oracle; then without the debug outputs (rows of at most 2048 keys
+    are not scored: other shares) and on a runtime of 4096 keys (a chunk a workgroup,
+    no shares), both bit for bit."""
+    edges = [4096, 2048, 2049, 1, 3072, 3073, 1024, 64, 4095, 2047, 2050]
+    ctx = [edges[(3 * i + i // 11) % 11] for i in range(rows)]
+    out, _, _ = _check(rt, ctx, 30 + rows, gpu_device)
+    step, caches = workloads.attn_case(ctx, gpu_device, seed=30 + rows)
+    plain = rt.forward(step, caches)
+    small = AttnRuntime(rows, 4096, device=gpu_device)
+    try:
+        one = small.forward(step, caches)
+        torch.cuda.synchronize()
+        small.check_errors()
+    finally:
+        small.close()
+    assert torch.equal(out, plain) and torch.equal(out, one)
+    # one long row among short ones: most workgroups' shares lie in that row
+    ctx = [5] * (rows - 2) + [32768, 2500]
+    out, _, _ = _check(rt, ctx, 60 + rows, gpu_device)
+    step, caches = workloads.attn_case(ctx, gpu_device, seed=60 + rows)
+    assert torch.equal(out, rt.forward(step, caches))
+
+
 @pytest.mark.parametrize("period", [1, 6])
 def test_attn_repeated_scores(rt, gpu_device, period):
     """Index planes whose pages repeat every `period` pages: each score recurs about

@@ -298,6 +298,34 @@ def test_layer_verify_chain_sees_its_own_draft_keys(gpu_device):
         assert torch.equal(il["topk_slots"][j, :n].cpu(), want), j
 
 
+def test_layer_verify_chain_of_a_wide_step(gpu_device):
+    """A verify chain of 12 rows at 4090 .. 4101 keys of 32768: the step's scored chunks
+    run in shares over the workgroups, and the keys that the step itself writes, on both
+    sides of a chunk boundary, are scored after the front wrote them: bit for bit what the
+    split launches give."""
+    ctx, rows = 32768, 12
+    cos, sin = workloads.rope_tables(ctx, gpu_device)
+    w = LayerWeights(proj=workloads.proj_weights(gpu_device, seed=61),
+                     moe=workloads.fp8_moe_weights(FP8_MOE, gpu_device, seed=62))
+    x = workloads.rows_bf16(rows, ol.HIDDEN, gpu_device, seed=64)
+    seq = torch.arange(4090, 4090 + rows, dtype=torch.int32, device=gpu_device)
+    got = {}
+    for mode in ("layer", "split"):
+        step, caches = workloads.attn_case([8192], gpu_device, seed=63, max_ctx=ctx)
+        pt = step.page_table[:1].repeat(rows, 1).contiguous()
+        rt = LayerRuntime(rows, ctx, gpu_device, mode=mode)
+        try:
+            got[mode] = rt.forward(x, seq, pt, caches, w, cos, sin, keep=True)
+            torch.cuda.synchronize()
+            rt.check_errors()
+        finally:
+            rt.close()
+    (xl, il), (xs, is_) = got["layer"], got["split"]
+    assert torch.equal(il["index_scores"], is_["index_scores"])
+    assert torch.equal(il["topk_slots"], is_["topk_slots"])
+    assert torch.equal(xl, xs)
+
+
 def test_layer_verify_chain_matches_oracle(gpu_device):
     """MTP verify rows past 2048 keys against the oracle (glm53/check.py:100-146):
     four rows of one request at positions 5118 .. 5121 (the chain crosses the 5120-key
