@@ -67,6 +67,10 @@ constexpr int AT = 512;
 constexpr int AW = AT / WAVE;
 constexpr int KPM = MAX_CTX / TMK;           // keys a top-k team member owns
 constexpr int KPT = KPM / AT;                // keys a thread of a member holds
+// a member that may hold a row alone stages its selected slots in LDS then and stores them
+// as one run (2048 slots, each thread storing its own: 4.3 us, staged 1.9; a member of a
+// team of 4, 512 slots: 1.2 and 1.8)
+constexpr bool kStageSel = KPM > TOPK;
 constexpr int SUB = 64;                      // tokens a split sub-tile
 constexpr int QK_HALF = DQK / 2;             // dims of q.k a wave sums (two waves a token tile)
 constexpr int QK_STEPS = QK_HALF / 32;       // its bf16 MFMA k steps
@@ -109,6 +113,7 @@ struct TopkLds {
   uint32_t tot[256];        // the team's
   uint32_t pre[256];        // the members' before this one
   uint32_t cu[CMAX];        // the team's threshold candidates, 0 past the last
+  int32_t sl[kStageSel ? TOPK : 1];  // this member's selected slots, in position order
   int32_t xw[TMK];          // the members' keys above the first digit
   int32_t cnt[TMK][2];      // the team's keys above / at the threshold
   uint32_t digit, uT;
@@ -303,7 +308,7 @@ class Step {
     // one sub-tile a split up to LONG_ROWS rows (its loop over sub-tiles compiles away),
     // long splits above, in k_attn_long alone (MONO_ATTN_LONG): every other launch takes
     // at most LONG_ROWS rows.
-    if (!kLongSplits || nsp == SPLITS) {
+    if (!kLongSplits) {
       for (T = first_at_or_after(base + n_topk); T < base + n_topk + n_split; T += G) {
         const uint64_t t0 = now_ticks();
         const int j = T - base - n_topk;
@@ -320,7 +325,7 @@ class Step {
         if (!ok) return false;
       }
     }
-    if (!kLongSplits || nsp == SPLITS) return merges<SPLITS, 1>(base + n_topk + n_split);
+    if (!kLongSplits) return merges<SPLITS, 1>(base + n_topk + n_split);
 #ifdef MONO_ATTN_WIDE
     return nsp == 8 ? merges<8, 4>(base + n_topk + n_split) : merges<4, 8>(base + n_topk + n_split);
 #else
@@ -724,12 +729,20 @@ class Step {
   // ---------------------------------------------------------------- top-k
   // exclusive prefix sum of v over the workgroup (a full barrier)
   MONO_DEV int block_excl_scan(int v) {
+    int total;
+    return block_excl_scan(v, total);
+  }
+  MONO_DEV int block_excl_scan(int v, int& total) {
     const int incl = wave_incl_scan(v);
     if (lane == WAVE - 1) L.scan[wave] = incl;
     __syncthreads();
     int before = 0;
+    total = 0;
 #pragma unroll
-    for (int w = 0; w < AW; ++w) before += w < wave ? L.scan[w] : 0;
+    for (int w = 0; w < AW; ++w) {
+      before += w < wave ? L.scan[w] : 0;
+      total += L.scan[w];
+    }
     __syncthreads();
     return before + incl - v;
   }
@@ -797,20 +810,44 @@ class Step {
     }
   }
 
+  // This member's keys under `prefix` counted by the digit at `shift` into an LDS histogram:
+  // plain atomics unless a quarter of the wave's first keys share the first lane's digit
+  // (ties: their atomics would serialize; hist_add takes those together, by a scalar chain
+  // a key: 8 rows of 32768 keys 31.9 -> 31.7 us a launch without it, 48 rows 71.1 -> 69.5)
+  MONO_DEV void hist_keys(uint32_t* hist, const uint32_t (&key)[KPT], int cnt, uint32_t prefix, uint32_t mask, int shift) {
+    cnt = opaque_v(cnt);  // (each pass over a thread's keys compares anew, see topk_member)
+    const uint32_t first = (key[0] >> shift) & 0xffu;
+    if (__popcll(__ballot(first == (uint32_t)__builtin_amdgcn_readfirstlane((int)first))) >= WAVE / 4) {  // wave-uniform
+#pragma unroll
+      for (int q = 0; q < KPT; ++q) hist_add(hist, q < cnt && (key[q] & mask) == prefix, (key[q] >> shift) & 0xffu);
+    } else {
+#pragma unroll
+      for (int q = 0; q < KPT; ++q)
+        if (q < cnt && (key[q] & mask) == prefix) atomicAdd(&hist[(key[q] >> shift) & 0xffu], 1u);
+    }
+  }
+
   // One exchanged radix pass: member m's histogram of the digit at `shift` over its keys
   // matching prefix under mask -> mailbox hist as 128 words of two 16-bit bins (a member
   // holds at most KPM keys), plus `count` as word 128 when count >= 0; the team's sum
   // -> K.tot, the sum over the members before m -> K.pre, the members' counts -> K.xw.
-  // Workgroup-uniform result.
-  MONO_DEV bool exchange_hist(int s, int m, int pass, const uint32_t (&key)[KPT], int cnt, uint32_t prefix,
+  // `lone`: the member holds the whole row. Workgroup-uniform result.
+  MONO_DEV bool exchange_hist(int s, int m, bool lone, int pass, const uint32_t (&key)[KPT], int cnt, uint32_t prefix,
                               uint32_t mask, int shift, int count) {
     static_assert(KPM < 65536, "16-bit bins");
     TopkLds& K = L.u.t;
     if (tid < 256) K.hist[tid] = 0u;
     __syncthreads();
-#pragma unroll
-    for (int q = 0; q < KPT; ++q) hist_add(K.hist, q < cnt && (key[q] & mask) == prefix, (key[q] >> shift) & 0xffu);
+    hist_keys(K.hist, key, cnt, prefix, mask, shift);
     __syncthreads();
+    if (lone) {  // team-uniform: nobody to exchange with
+      if (tid < 256) {
+        K.tot[tid] = K.hist[tid];
+        K.pre[tid] = 0u;
+      }
+      __syncthreads();
+      return true;
+    }
     uint64_t* hb = &A.mail.hist[((size_t)s * PASSES + pass) * TMK * HW];
     bool ok = true;
     if (tid < 128) {
@@ -852,7 +889,8 @@ class Step {
   // key bits, position) and every member ranks them all; a crowded threshold bin
   // instead takes digits 3 and 4 the same way as digit 2 and then the members' counts
   // above / at the threshold (mailbox cnt). Each member writes its selected slots at
-  // its offset in position order.
+  // its offset in position order. A row that its first member holds alone exchanges
+  // nothing (33 rows of 1500-12000 keys: 4.3 us of 16.5 a lone member's selection took).
   MONO_DEV bool topk_member(int s, int m) {
     TopkLds& K = L.u.t;
     const int n = row_len(s);
@@ -865,6 +903,8 @@ class Step {
       }
       return true;
     }
+    const bool lone = kStageSel && n <= KPM;
+    if (lone && m > 0) return true;
     const int p0 = m * KPM + tid * KPT;
     const int cnt = min(max(n - p0, 0), KPT);
     const int page = cnt > 0 ? page_of(s, p0) : 0;  // a thread's keys share one page
@@ -896,16 +936,22 @@ class Step {
     int need = TOPK - K.above;
     const uint32_t d1 = K.digit;
     uint32_t prefix = d1 << 24, mask = 0xff000000u;
+    // Each pass over a thread's keys compares its positions and keys anew (opaque copies):
+    // shared between the passes, KPT lane masks a comparison would be held in scalar
+    // registers and spilled
     int above1 = 0;  // this member's keys above digit 1
+    {
+      const int cn = opaque_v(cnt);
 #pragma unroll
-    for (int q = 0; q < KPT; ++q) above1 += (q < cnt && (key[q] >> 24) > d1) ? 1 : 0;
+      for (int q = 0; q < KPT; ++q) above1 += (q < cn && (key[q] >> 24) > d1) ? 1 : 0;
+    }
     above1 = wave_sum_i(above1);
     if (lane == 0) L.scan[wave] = above1;
     __syncthreads();
     above1 = 0;
 #pragma unroll
     for (int w = 0; w < AW; ++w) above1 += L.scan[w];
-    if (!exchange_hist(s, m, 1, key, cnt, prefix, mask, 16, above1)) return false;
+    if (!exchange_hist(s, m, lone, 1, key, cnt, prefix, mask, 16, above1)) return false;
     pick_digit(K, K.tot, need, K.pre);
     __syncthreads();
     need -= K.above;
@@ -923,19 +969,33 @@ class Step {
     if (cand) {
       const uint32_t P16 = prefix >> 16;
       int c_my = 0;
+      {
+        const int cn = opaque_v(cnt);
 #pragma unroll
-      for (int q = 0; q < KPT; ++q) c_my += (q < cnt && (key[q] >> 16) == P16) ? 1 : 0;
+        for (int q = 0; q < KPT; ++q) c_my += (q < cn && (key[q] >> 16) == P16) ? 1 : 0;
+      }
+      static_assert(CMAX == AT, "a thread a candidate");
+      if (lone) K.cu[tid] = 0u;
       int idx = cand_before + block_excl_scan(c_my);
       uint64_t* cb = &A.mail.cand[(size_t)s * CMAX];
-#pragma unroll
-      for (int q = 0; q < KPT; ++q)
-        if (q < cnt && (key[q] >> 16) == P16) mb_put(&cb[idx++], cand_word(key[q], p0 + q), gd.tag);
-      static_assert(CMAX == AT, "a thread a candidate");
       uint32_t u = 0;
       ok = true;
-      if (tid < n_cand) ok = poll_word(&cb[tid], u, W_TEAM, gd);
-      K.cu[tid] = u;
-      if (!block_all(ok)) return false;
+      const int cn = opaque_v(cnt);
+      const uint32_t P16b = (uint32_t)opaque_v((int)P16);
+      if (lone) {
+#pragma unroll
+        for (int q = 0; q < KPT; ++q)
+          if (q < cn && (key[q] >> 16) == P16b) K.cu[idx++] = cand_word(key[q], p0 + q);
+        __syncthreads();
+        u = K.cu[tid];
+      } else {
+#pragma unroll
+        for (int q = 0; q < KPT; ++q)
+          if (q < cn && (key[q] >> 16) == P16b) mb_put(&cb[idx++], cand_word(key[q], p0 + q), gd.tag);
+        if (tid < n_cand) ok = poll_word(&cb[tid], u, W_TEAM, gd);
+        K.cu[tid] = u;
+        if (!block_all(ok)) return false;
+      }
       if (wave * WAVE < n_cand) {  // wave-uniform
         // candidates ranked before this thread's, 32 a step with the step's LDS reads issued
         // together (K.cu holds zeros past the last candidate, and a step starting below
@@ -960,7 +1020,7 @@ class Step {
       for (int pass = 2; pass < PASSES; ++pass) {
         const int shift = 24 - 8 * pass;
         __syncthreads();  // K.digit and K.tot are read
-        if (!exchange_hist(s, m, pass, key, cnt, prefix, mask, shift, -1)) return false;
+        if (!exchange_hist(s, m, lone, pass, key, cnt, prefix, mask, shift, -1)) return false;
         pick_digit(K, K.tot, need, nullptr);
         __syncthreads();
         need -= K.above;
@@ -980,7 +1040,7 @@ class Step {
         mb_put(&A.mail.cnt[((size_t)s * TMK + m) * 2 + 1], (uint32_t)(eq_in + c_eq), gd.tag);
       }
       ok = true;
-      if (tid < 2 * TMK) {
+      if (tid < 2 * (lone ? 1 : TMK)) {
         uint32_t v = 0;
         ok = poll_word(&A.mail.cnt[(size_t)s * TMK * 2 + tid], v, W_TEAM, gd);
         K.cnt[tid / 2][tid % 2] = (int)v;
@@ -998,24 +1058,43 @@ class Step {
     }
     // the selected keys in position order: above the threshold prefix, and the
     // threshold's share (candidates ranked at or above uT / the first uT equal to T)
-    bool take[KPT];
-    int c_take = 0, te = 0;
-#pragma unroll
-    for (int q = 0; q < KPT; ++q) {
+    uint32_t take = 0;  // bit q: key q is selected
+    {
+      const int cn = opaque_v(cnt);
       if (cand) {
-        const uint32_t hi = key[q] >> 16;
-        take[q] = q < cnt && (hi > (prefix >> 16) || (hi == (prefix >> 16) && cand_word(key[q], p0 + q) >= uT));
-      } else {
-        const bool eq = q < cnt && key[q] == prefix;
-        take[q] = (q < cnt && key[q] > prefix) || (eq && te < (int)uT);
-        te += eq ? 1 : 0;
-      }
-      c_take += take[q] ? 1 : 0;
-    }
-    int idx = sel_before + block_excl_scan(c_take);
 #pragma unroll
-    for (int q = 0; q < KPT; ++q)
-      if (take[q] && idx < TOPK) publish_sel(s, idx++, page * PAGE + (p0 + q) % PAGE);
+        for (int q = 0; q < KPT; ++q) {
+          const uint32_t hi = key[q] >> 16, P16 = prefix >> 16;
+          const bool t = q < cn && (hi > P16 || (hi == P16 && cand_word(key[q], p0 + q) >= uT));
+          take |= t ? 1u << q : 0u;
+        }
+      } else {
+        int te = 0;
+#pragma unroll
+        for (int q = 0; q < KPT; ++q) {
+          const bool eq = q < cn && key[q] == prefix;
+          const bool t = (q < cn && key[q] > prefix) || (eq && te < (int)uT);
+          te += eq ? 1 : 0;
+          take |= t ? 1u << q : 0u;
+        }
+      }
+    }
+    const int c_take = __popc(take);
+    if (kStageSel && lone) {
+      int n_sel;
+      int idx = block_excl_scan(c_take, n_sel);
+#pragma unroll
+      for (int q = 0; q < KPT; ++q)
+        if ((take >> q & 1u) && idx < TOPK) K.sl[idx++] = page * PAGE + (p0 + q) % PAGE;
+      __syncthreads();
+      for (int j = tid; j < n_sel && sel_before + j < TOPK; j += AT) publish_sel(s, sel_before + j, K.sl[j]);
+      __syncthreads();  // the next task may rewrite the LDS
+    } else {
+      int idx = sel_before + block_excl_scan(c_take);
+#pragma unroll
+      for (int q = 0; q < KPT; ++q)
+        if ((take >> q & 1u) && idx < TOPK) publish_sel(s, idx++, page * PAGE + (p0 + q) % PAGE);
+    }
     return true;
   }
 

@@ -152,6 +152,15 @@ def test_attn_score_runs(rt, gpu_device, rows):
     assert torch.equal(out, rt.forward(step, caches))
 
 
+@pytest.mark.parametrize("period", [0, 1, 6])
+def test_attn_rows_of_one_member(rt, gpu_device, period):
+    """Wide steps whose rows fit one top-k member (at most 8192 keys) beside rows that take
+    two and four: no exchange in the former, with spread scores (threshold candidates
+    ranked in place) and with repeated ones (digits 3 and 4, ties to the lowest position)."""
+    ctx = ([2049, 8192, 8193, 4000, 2048, 16400, 8191, 32768] * 3)[:20]
+    _check(rt, ctx, 50 + period, gpu_device, period=period)
+
+
 @pytest.mark.parametrize("period", [1, 6])
 def test_attn_repeated_scores(rt, gpu_device, period):
     """Index planes whose pages repeat every `period` pages: each score recurs about
