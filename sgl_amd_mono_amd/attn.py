@@ -24,14 +24,14 @@ IH, ID, NH, DQK, DV, PAGE, TOPK = 64, 128, 32, 576, 512, 64, 2048
 
 
 def splits_of(rows: int) -> int:
-    """Attention splits a row: 32 up to 16 rows, then fewer and longer ones, so a step's
-    splits fill one round of a 256-CU grid."""
-    return 32 if rows <= 16 else 8 if rows <= 32 else 5 if rows <= 48 else 4
+    """Attention splits a row: 32 up to 16 rows; above, the launch shares the step's selected
+    tokens out over at most 256 splits (this many a row on average, at most)."""
+    return 32 if rows <= 16 else -(-256 // rows)
 
 
 def merges_of(rows: int) -> int:
-    """Merge tasks a row (32 / merges heads each): as many as splits, except 4 with 5."""
-    return 4 if splits_of(rows) == 5 else splits_of(rows)
+    """Merge tasks a row (32 / merges heads each)."""
+    return 32 if rows <= 16 else 8 if rows <= 32 else 4
 SOFTMAX_SCALE = (128 + 64) ** -0.5  # (qk_nope + qk_rope)^-1/2, glm53/gfx950/config.py:171-173
 
 

@@ -67,9 +67,9 @@ constexpr int AT = 512;
 constexpr int AW = AT / WAVE;
 constexpr int KPM = MAX_CTX / TMK;           // keys a top-k team member owns
 constexpr int KPT = KPM / AT;                // keys a thread of a member holds
-// a member that may hold a row alone stages its selected slots in LDS then and stores them
-// as one run (2048 slots, each thread storing its own: 4.3 us, staged 1.9; a member of a
-// team of 4, 512 slots: 1.2 and 1.8)
+// a member of many keys stages its selected slots in LDS and stores them as one run: each
+// thread storing its own took 4.3 us for a member that holds its row alone (staged 1.9; 33
+// rows of 1500-12000 keys 44.2 -> 43.1 us a launch, 48 rows of 32768 71.0 -> 70.1)
 constexpr bool kStageSel = KPM > TOPK;
 constexpr int SUB = 64;                      // tokens a split sub-tile
 constexpr int QK_HALF = DQK / 2;             // dims of q.k a wave sums (two waves a token tile)
@@ -108,7 +108,6 @@ struct ScoreLds {
 };
 
 struct TopkLds {
-  int32_t pt[TOPK / PAGE];  // a short row's page table
   uint32_t hist[256];       // this member's digit histogram
   uint32_t tot[256];        // the team's
   uint32_t pre[256];        // the members' before this one
@@ -290,15 +289,14 @@ class Step {
   template <class Between>
   MONO_DEV bool tasks(Between&& between) {
     const int n_topk = A.rows * TMK;
-    const int nsp = splits_of(A.rows);
-    const int n_split = A.rows * nsp;
+    if (kLongSplits || A.rows * CH > G) row_n = lane < A.rows ? row_len(lane) : 0;
     if (!scores()) return false;
     // a workgroup's list is ordered by stage: one loop a stage keeps each loop body to
     // one task kind (and its registers). The list after the scores starts at `base` (a
     // multiple of TMK); a task's timeline row is its list index + tl0.
-    const int tl0 = n_score() - base;
+    const int tl0 = n_score() - base, at = base + n_topk;
     int T = first_at_or_after(base);
-    for (; T < base + n_topk; T += G) {
+    for (; T < at; T += G) {
       const uint64_t t0 = now_ticks();
       const bool ok = topk_member((T - base) / TMK, (T - base) % TMK);
       stamp(T + tl0, t0, 1);
@@ -306,32 +304,28 @@ class Step {
     }
     if (!between()) return false;
     // one sub-tile a split up to LONG_ROWS rows (its loop over sub-tiles compiles away),
-    // long splits above, in k_attn_long alone (MONO_ATTN_LONG): every other launch takes
-    // at most LONG_ROWS rows.
-    if (!kLongSplits) {
-      for (T = first_at_or_after(base + n_topk); T < base + n_topk + n_split; T += G) {
-        const uint64_t t0 = now_ticks();
-        const int j = T - base - n_topk;
-        const bool ok = split_task<false>(j / SPLITS, j % SPLITS, SPLITS);
+    // splits of the plan above, in k_attn_long alone (MONO_ATTN_LONG): every other launch
+    // takes at most LONG_ROWS rows.
+    const int n_split = kLongSplits ? first_split(A.rows) : A.rows * SPLITS;
+    for (T = first_at_or_after(at); T < at + n_split; T += G) {
+      const uint64_t t0 = now_ticks();
+      const int i = T - at;
+      bool ok;
+      if (kLongSplits) {
+        const int s = (int)__popcll(__ballot(sp_inc <= i)), j = i - first_split(s);
+        const int nst = sub_tiles(__builtin_amdgcn_readlane(row_n, s)), nsp = first_split(s + 1) - first_split(s);
+        const int rcp = recip(nsp), lo = j * nst * rcp >> 16, hi = (j + 1) * nst * rcp >> 16;
+        ok = split_task<true>(s, j, lo * SUB, (hi - lo) * SUB);
+        if (i < A.rows * splits_of(A.rows)) stamp(T + tl0, t0, 2);
+      } else {
+        ok = split_task<false>(i / SPLITS, i % SPLITS, i % SPLITS * SUB, SUB);
         stamp(T + tl0, t0, 2);
-        if (!ok) return false;
       }
-    } else {
-      for (T = first_at_or_after(base + n_topk); T < base + n_topk + n_split; T += G) {
-        const uint64_t t0 = now_ticks();
-        const int j = T - base - n_topk;
-        const bool ok = split_task<true>(j / nsp, j % nsp, nsp);
-        stamp(T + tl0, t0, 2);
-        if (!ok) return false;
-      }
+      if (!ok) return false;
     }
-    if (!kLongSplits) return merges<SPLITS, 1>(base + n_topk + n_split);
-#ifdef MONO_ATTN_WIDE
-    return nsp == 8 ? merges<8, 4>(base + n_topk + n_split) : merges<4, 8>(base + n_topk + n_split);
-#else
-    if (nsp == 8) return merges<8, 4>(base + n_topk + n_split);
-    return nsp == 5 ? merges<5, 8>(base + n_topk + n_split) : merges<4, 8>(base + n_topk + n_split);
-#endif
+    const int tlm = n_score() + n_topk + A.rows * splits_of(A.rows);
+    if (!kLongSplits) return merges<1>(at + n_split, tlm);
+    return merges_of(A.rows) == 8 ? merges<4>(at + n_split, tlm) : merges<8>(at + n_split, tlm);
   }
 
  private:
@@ -340,9 +334,34 @@ class Step {
   Guard gd;
   int tid, lane, wave, g, r, G, CH;
   int base = 0;
+  int row_n = 0;   // lane s: row s's length (wide steps)
+  int sp_inc = 0;  // lane s: the splits of rows 0 .. s (k_attn_long)
   bool q_ready = false;  // the front's q has been awaited (a fused launch)
   uint64_t waited = 0;
 
+  // sub-tiles of selected tokens of a row of n keys
+  MONO_DEV static int sub_tiles(int n) { return (min(n, TOPK) + SUB - 1) / SUB; }
+  // The splits of a wide step: as few sub-tiles a split (sp) as let the step's splits fit
+  // one round of the grid; row s has ceil(its sub-tiles / sp) splits of even length. A
+  // fixed count a row (8 to 32 rows, 5 to 48, 4 above) gave 33 rows splits of 7 sub-tiles
+  // where 5 fit, 17 rows 4 where 3 fit, and a short row's first splits as much as they held
+  // (33 rows of 1500-12000 keys: 47.9 -> 42.6 us a launch). Taken while the first keys are
+  // on their way.
+  MONO_DEV void plan_splits() {
+    const int nst = sub_tiles(row_n);
+    const int total = wave_incl_scan(nst);
+    int sp = 1;  // at least the even share
+    for (int left = __builtin_amdgcn_readlane(total, WAVE - 1) - G; left > 0 && sp < SPLIT_MAX / SUB; left -= G) ++sp;
+#pragma unroll 1
+    for (;; ++sp) {
+      sp_inc = wave_incl_scan((nst + sp - 1) * recip(sp) >> 16);
+      if (sp == SPLIT_MAX / SUB || __builtin_amdgcn_readlane(sp_inc, WAVE - 1) <= G) break;
+    }
+  }
+  // x * recip(d) >> 16 == x / d for 1 <= d <= 32 and 0 <= x <= 1024 (a reciprocal rounded up)
+  MONO_DEV static int recip(int d) { return (int)(65536.0f * hw_rcp((float)d)) + 1; }
+  // the list index (from the first split) of row s's first split
+  MONO_DEV int first_split(int s) const { return s > 0 ? __builtin_amdgcn_readlane(sp_inc, s - 1) : 0; }
   // a row's chunks that are scored
   MONO_DEV int live_chunks(int n) const { return n > TOPK || A.scores ? (n + CHUNK - 1) / CHUNK : 0; }
   MONO_DEV int row_len(int s) const { return min(max(A.seq_lens[s], 0), A.mail.max_ctx); }
@@ -568,6 +587,7 @@ class Step {
       // a workgroup for every chunk of max_ctx: chunk b, with no look at the other rows'
       // lengths in front of its loads (a round trip, ~1 us at 8 rows)
       base = n_score();
+      if (kLongSplits) plan_splits();
       const int b = block_index();
       if (b < A.rows * CH) {
         const int s = b / CH, c = b % CH, n = row_len(s);
@@ -618,18 +638,21 @@ class Step {
   // the launch 76.0 -> 70.5).
   MONO_DEV bool score_run() {
     ScoreLds& P = L.u.sc;
-    const int nl = lane < A.rows ? row_len(lane) : 0;
+    const int nl = row_n;
     const int inc = wave_incl_scan(live_chunks(nl));
     const int total = __builtin_amdgcn_readlane(inc, WAVE - 1), b = block_index();
     base = (min(total, G) + TMK - 1) / TMK * TMK;
     int i0 = total > G ? (int)((int64_t)b * total / G) : min(b, total);
     const int i1 = total > G ? (int)((int64_t)(b + 1) * total / G) : min(b + 1, total);
-    if (i0 >= i1) return true;  // workgroup-uniform
+    if (i0 >= i1) {  // workgroup-uniform
+      if (kLongSplits) plan_splits();
+      return true;
+    }
     if (tid < 256) P.hist[tid] = 0u;
     // row s of scored chunk i, and the row's first one
     const auto row_at = [inc](int i) { return (int)__popcll(__ballot(inc <= i)); };
     const auto first_of = [inc](int s) { return s > 0 ? __builtin_amdgcn_readlane(inc, s - 1) : 0; };
-    bool awaited = !front_here();
+    bool awaited = !front_here(), planned = !kLongSplits;
 #pragma unroll 1
     for (; i0 < i1; i0 += RUN) {
       const Lane z = lane_now();
@@ -657,6 +680,8 @@ class Step {
       if (awaited) {
         key_load(z, ka, pages_of(z, 0));
         key_load(z, kb, pages_of(z, 1));
+        if (!planned) plan_splits();
+        planned = true;
       } else {
         const auto fresh_at = [&](int j) {
           const int sj = row_at(i0 + min(j, m - 1));
@@ -894,13 +919,9 @@ class Step {
   MONO_DEV bool topk_member(int s, int m) {
     TopkLds& K = L.u.t;
     const int n = row_len(s);
-    if (n <= TOPK) {  // every key is selected; no score is needed
-      if (m == 0) {
-        for (int i = tid; i < TOPK / PAGE; i += AT) K.pt[i] = i * PAGE < n ? page_of(s, i * PAGE) : 0;
-        __syncthreads();
-        for (int j = tid; j < TOPK; j += AT) publish_sel(s, j, j < n ? K.pt[j / PAGE] * PAGE + j % PAGE : -1);
-        __syncthreads();  // the next task may rewrite the LDS page table
-      }
+    if (n <= TOPK) {  // every key is selected, in place (split_task); only a caller's copy is written here
+      if (A.topk && m == 0)
+        for (int j = tid; j < TOPK; j += AT) A.topk[(size_t)s * TOPK + j] = j < n ? slot_of(s, j) : -1;
       return true;
     }
     const bool lone = kStageSel && n <= KPM;
@@ -1080,7 +1101,7 @@ class Step {
       }
     }
     const int c_take = __popc(take);
-    if (kStageSel && lone) {
+    if (kStageSel) {
       int n_sel;
       int idx = block_excl_scan(c_take, n_sel);
 #pragma unroll
@@ -1091,9 +1112,17 @@ class Step {
       __syncthreads();  // the next task may rewrite the LDS
     } else {
       int idx = sel_before + block_excl_scan(c_take);
+      // (a key not taken stores past the row's words: the buffer drops it, no branch a key;
+      // 8 rows of 32768 keys: 31.4 -> 31.3 us a launch)
+      const __amdgpu_buffer_rsrc_t rs = coherent_rsrc(A.mail.sel + (size_t)s * TOPK, TOPK * 8);
 #pragma unroll
-      for (int q = 0; q < KPT; ++q)
-        if ((take >> q & 1u) && idx < TOPK) publish_sel(s, idx++, page * PAGE + (p0 + q) % PAGE);
+      for (int q = 0; q < KPT; ++q) {
+        const bool t = take >> q & 1u;
+        const u32x2 w = {(uint32_t)(page * PAGE + (p0 + q) % PAGE), gd.tag};
+        __builtin_amdgcn_raw_buffer_store_b64(w, rs, t ? idx * 8 : TOPK * 8, 0, SC1);
+        if (A.topk && t && idx < TOPK) A.topk[(size_t)s * TOPK + idx] = (int)w[0];
+        idx += t ? 1 : 0;
+      }
     }
     return true;
   }
@@ -1133,39 +1162,41 @@ class Step {
     }
   }
 
+  // Every slot of sub-tile st is a cached row (wave-uniform): no row to clear, no token to
+  // leave out (all but a row's last sub-tile; 30 of a thread's ~400 VALU a sub-tile).
+  MONO_DEV bool sub_full(const SplitLds& P, int st) const { return __ballot(P.slot[st * SUB + lane] < 0) == 0; }
+
   // Store sub-tile st's rows into its buffer as they lie, the rows of empty slots as
   // zeros, and its scales. One copy serves q.k and p.v: a second, widened and transposed
   // one (64 KB of LDS stores, 64 VALU a thread and two more barriers a sub-tile) put 0.7
   // us on the chain of a one-sub-tile split (one row of 700 keys: 13.2 -> 12.5 us a launch).
   MONO_DEV void gather_store(SplitLds& P, int st, const Gather& gt) {
+    if (sub_full(P, st))
+      gather_store_rows<true>(P, st, gt);
+    else
+      gather_store_rows<false>(P, st, gt);
+  }
+  template <bool FULL>
+  MONO_DEV void gather_store_rows(SplitLds& P, int st, const Gather& gt) {
     const int c = tid % (DV / 16), m = tid / (DV / 16);
     const int32_t* sl = P.slot + st * SUB;
     u32x4(*kf)[KF_W / 4] = P.kf16[st % 2];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) kf[4 * m + k][c] = sl[4 * m + k] >= 0 ? gt.v[k] : u32x4{0u, 0u, 0u, 0u};
+    for (int k = 0; k < 4; ++k) kf[4 * m + k][c] = FULL || sl[4 * m + k] >= 0 ? gt.v[k] : u32x4{0u, 0u, 0u, 0u};
     if (tid < ROPE_CH * SUB) {
       const int t = tid / ROPE_CH;
-      kf[t][DV / 16 + tid % ROPE_CH] = sl[t] >= 0 ? gt.rope : u32x4{0u, 0u, 0u, 0u};
+      kf[t][DV / 16 + tid % ROPE_CH] = FULL || sl[t] >= 0 ? gt.rope : u32x4{0u, 0u, 0u, 0u};
     }
-    if (tid < SUB) P.kvs[st % 2][tid] = sl[tid] >= 0 ? gt.sc : 0.f;
+    if (tid < SUB) P.kvs[st % 2][tid] = FULL || sl[tid] >= 0 ? gt.sc : 0.f;
   }
 
-  // Split j of row s's nsp: its selected tokens in sub-tiles of SUB, [32 j / nsp, 32 (j +
-  // 1) / nsp) of the row's 32. LONG: a split may hold several sub-tiles (fewer than
-  // SPLITS splits a row).
+  // Split j of row s: its selected tokens lo .. lo + len - 1 (whole sub-tiles of SUB). LONG:
+  // a split may hold several sub-tiles.
   template <bool LONG>
-  MONO_DEV bool split_task(int s, int j, int nsp) {
+  MONO_DEV bool split_task(int s, int j, int lo, int len) {
     SplitLds& P = L.u.sp;
-    const int nsel = min(row_len(s), TOPK);
-#ifdef MONO_ATTN_WIDE
-    const int len = LONG ? TOPK / nsp : TOPK / SPLITS;  // 4 even splits a row
-    const int lo = j * len;
-#else
-    constexpr int NST = TOPK / SUB;  // sub-tiles a row
-    const int lo = LONG ? (j * NST / nsp) * SUB : j * (TOPK / SPLITS);
-    const int len = LONG ? ((j + 1) * NST / nsp) * SUB - lo : TOPK / SPLITS;
-#endif
-    const int cnt = min(max(nsel - lo, 0), len);
+    const int n = row_len(s);
+    const int cnt = min(max(min(n, TOPK) - lo, 0), len);
     const size_t mlb = ((size_t)s * SPLITS + j) * NH;
     if (cnt == 0) {  // an empty split contributes nothing to the merge
       if (tid < NH) {
@@ -1175,9 +1206,13 @@ class Step {
       split_done(s, j);
       return true;
     }
-    if (front_here() && !q_ready) {  // every head of q from the front of this launch
-      const uint64_t* fd = done_copy(A.fdone) + proj::FD_D;
-      if (!hint_wait(NH, [fd](int i) { return fd + i; }, A.fsite + 1, gd)) return false;
+    if (front_here() && !q_ready) {
+      // every head of q from the front of this launch, and every row's cache row (a row that
+      // selects all its keys waits for no scores, which would follow them)
+      const uint64_t* fd = done_copy(A.fdone);
+      if (!hint_wait(NH + A.rows, [fd](int i) { return fd + (i < NH ? proj::FD_D + i : proj::FD_B + i - NH); },
+                     A.fsite + 1, gd))
+        return false;
       q_ready = true;
     }
     {
@@ -1194,7 +1229,11 @@ class Step {
     bool ok = true;
     if (tid < len) {
       int slot = -1;
-      if (tid < cnt) {
+      if (tid < cnt && n <= TOPK) {
+        // every key of the row is selected: no selection to wait for (one row of 700 keys:
+        // 12.3 -> 11.9 us a launch)
+        slot = slot_of(s, lo + tid);
+      } else if (tid < cnt) {
         uint32_t v = 0;
         ok = poll_word(&A.mail.sel[(size_t)s * TOPK + lo + tid], v, W_SEL, gd);
         slot = (int)v;
@@ -1262,22 +1301,28 @@ class Step {
       {
         const int ti = LONG ? opaque_v(tid) : tid, h = ti / 16, tq = ti % 16;
         const f32x4 x0 = P.pf4[0][h][tq], x1 = P.pf4[1][h][tq], ks = P.kvs4[buf][tq];
-        const i32x4 sl = P.slot4[st * (SUB / 4) + tq];
         float x[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = sl[i] >= 0 ? (x0[i] + x1[i]) * (ks[i] * A.scale) : NEG_INF;
-        const float mx = fmaxf(m_run, row_reduce<16>(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), OpMax()));
+        for (int i = 0; i < 4; ++i) x[i] = (x0[i] + x1[i]) * (ks[i] * A.scale);
+        if (!sub_full(P, st)) {
+          const i32x4 sl = P.slot4[st * (SUB / 4) + tq];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[i] = sl[i] >= 0 ? x[i] : NEG_INF;
+        }
+        float mx = row_reduce<16>(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), OpMax());
+        if (LONG) mx = fmaxf(m_run, mx);
         float pr[4], ps = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           pr[i] = (mx == NEG_INF || x[i] == NEG_INF) ? 0.f : hw_exp(x[i] - mx);
           ps += pr[i];
         }
+        ps = row_reduce<16>(ps, OpAdd());
         const float al = m_run == NEG_INF ? (mx == NEG_INF ? 1.f : 0.f) : hw_exp(m_run - mx);
-        l_run = l_run * al + row_reduce<16>(ps, OpAdd());
+        l_run = LONG ? l_run * al + ps : ps;
         m_run = mx;
         P.pb8[h][tq] = u32x2{pack_bf16x2(pr[0] * ks[0], pr[1] * ks[1]), pack_bf16x2(pr[2] * ks[2], pr[3] * ks[3])};
-        if (tq == 0) P.alpha[h] = al;
+        if (LONG && tq == 0) P.alpha[h] = al;
       }
       // the next sub-tile's rows into the other buffer (its last readers, the p.v of the
       // sub-tile before, are behind this phase's first barrier) and the rows after them
@@ -1291,15 +1336,17 @@ class Step {
       // one dim of the 8 tokens) and widened, B = 16 heads' probabilities, k = 32 tokens
       // a step
       {
-        float alh[2];
+        if (LONG) {
+          float alh[2];
 #pragma unroll
-        for (int a = 0; a < 2; ++a) alh[a] = P.alpha[16 * a + r];
+          for (int a = 0; a < 2; ++a) alh[a] = P.alpha[16 * a + r];
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+          for (int b = 0; b < 4; ++b)
 #pragma unroll
-          for (int a = 0; a < 2; ++a)
+            for (int a = 0; a < 2; ++a)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[b][a][i] *= alh[a];
+              for (int i = 0; i < 4; ++i) acc[b][a][i] *= alh[a];
+        }
 #pragma unroll
         for (int kt = 0; kt < SUB / 32; ++kt) {
           bf16x8 pv[2], va[4];  // every operand of the k step read before its MFMAs
@@ -1363,89 +1410,120 @@ class Step {
   }
 
   // ---------------------------------------------------------------- merge
-  // This workgroup's merges over a row's NSP splits: list index `at` + k is merge k (row
+  // This workgroup's merges: list index `at` + k (timeline row tl + k) is merge k (row
   // k / (32 / HM), heads (k % (32 / HM)) HM ..), HM heads a task.
-  template <int NSP, int HM>
-  MONO_DEV bool merges(int at) {
-    constexpr int MPR = SPLITS / HM;  // merges a row
+  template <int HM>
+  MONO_DEV bool merges(int at, int tl) {
+    constexpr int MPR = NH / HM;  // merges a row
     const int n = A.rows * MPR;
     for (int T = first_at_or_after(at); T < at + n; T += G) {
       const uint64_t t0 = now_ticks();
-      const int k = T - at;
-      const bool ok = merge_task<NSP, HM>(k / MPR, k % MPR);
-      stamp(T + n_score() - base, t0, 3);
+      const int k = T - at, s = k / MPR;
+      const bool ok = merge_task<HM>(s, k % MPR, kLongSplits ? first_split(s + 1) - first_split(s) : SPLITS);
+      stamp(tl + k, t0, 3);
       if (!ok) return false;
     }
     return true;
   }
 
-  // Merge (row s, heads hg HM .. hg HM + HM - 1) over the row's NSP splits: each thread
-  // combines IPT channel pairs (a task takes in NSP x HM KB of partials, 32 or 40 KB).
-  template <int NSP, int HM>
-  MONO_DEV bool merge_task(int s, int hg) {
-    constexpr int ITEMS = HM * DV / 2;                // channel pairs of the task
-    constexpr int IPT = ITEMS > AT ? ITEMS / AT : 1;  // pairs a thread
-    static_assert(NSP <= WAVE && HM <= AW && HM <= 8 && (ITEMS % AT == 0 || ITEMS < AT) && NH % HM == 0,
+  // N dwords at uniform offset `u` plus lane offset `v` of a device-coherent resource
+  template <int N>
+  MONO_DEV static void load_words(__amdgpu_buffer_rsrc_t rs, int v, int u, uint32_t (&w)[N]) {
+    if constexpr (N == 4) {
+      const u32x4 x = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, v, u, SC1));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = x[i];
+    } else if constexpr (N == 2) {
+      const u32x2 x = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, v, u, SC1));
+      w[0] = x[0];
+      w[1] = x[1];
+    } else {
+      static_assert(N == 1, "4, 8 or 16 bytes");
+      w[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_raw_buffer_load_b32(rs, v, u, SC1));
+    }
+  }
+
+  // Merge (row s, heads hg HM .. hg HM + HM - 1) over the row's nsp splits: each thread
+  // combines CPT consecutive channels of a head, BATCH splits at a time (a task takes in
+  // nsp x HM KB of partials, by loads of up to 16 bytes).
+  template <int HM>
+  MONO_DEV bool merge_task(int s, int hg, int nsp) {
+    constexpr int CPT = HM > 2 ? HM : 2;  // channels a thread
+    constexpr int BATCH = kLongSplits ? 8 : SPLITS;
+    static_assert(SPLITS <= WAVE && HM <= AW && HM <= 8 && HM * DV / CPT <= AT && NH % HM == 0,
                   "a lane a split; a wave a head's weights");
     MergeLds& Q = L.u.mg;
     const int h0 = hg * HM;
     const size_t rb = (size_t)s * SPLITS;
     // every split of the row done: lane j of wave 0 polls split j's word
     bool ok = true;
-    if (wave == 0 && lane < NSP) {
+    if (wave == 0 && lane < nsp) {
       uint32_t v;
       ok = poll_word(&A.mail.sdone[rb + lane], v, W_PART, gd);
     }
     if (!block_all(ok)) return false;
     mark_waited();
-    // the split weights: wave w takes head h0 + w, lane j split j
+    // the split weights: wave w takes head h0 + w, lane j split j (0 past the last)
     if (wave < HM) {
       const int h = h0 + wave;
-      const int jl = min(lane, NSP - 1);
+      const int jl = max(min(lane, nsp - 1), 0);
       const float m = ld_agent_f32(&A.mail.ml[((rb + jl) * NH + h) * 2]);
-      const float l = lane < NSP ? ld_agent_f32(&A.mail.ml[((rb + jl) * NH + h) * 2 + 1]) : 0.f;
+      const float l = lane < nsp ? ld_agent_f32(&A.mail.ml[((rb + jl) * NH + h) * 2 + 1]) : 0.f;
       const bool live = l > 0.f;
       const float M = wave_max(live ? m : NEG_INF);
       const float w = live ? hw_exp(m - M) : 0.f;
       const float den = wave_sum(w * l);
-      if (lane < NSP) Q.w[wave][lane] = w;
+      if (lane < SPLITS) Q.w[wave][lane] = w;
       if (lane == 0) Q.den[wave] = den;
     }
-    // the channel pairs of every split (unconditional loads; an empty split's words are
+    // the channels of the batch's splits (unconditional loads; an empty split's words are
     // read and ignored)
-    const bool mine = tid < ITEMS;  // wave-uniform
-    uint32_t av[IPT][NSP];
-    if (mine) {
+    const int c0 = tid * CPT, hh = c0 / DV;  // channel of the task's HM heads, its head
+    const bool mine = c0 < HM * DV;          // wave-uniform
+    const __amdgpu_buffer_rsrc_t rs = coherent_rsrc(A.mail.part + rb * NH * DV, SPLITS * NH * DV * 2);
+    float o[CPT];
 #pragma unroll
-      for (int k = 0; k < IPT; ++k) {
-        const int it = tid + AT * k, h = h0 + it / (DV / 2), d0 = (it % (DV / 2)) * 2;
+    for (int i = 0; i < CPT; ++i) o[i] = 0.f;
+    uint32_t av[BATCH][CPT / 2];
+    const auto load = [&](int j0) {
 #pragma unroll
-        for (int j = 0; j < NSP; ++j)
-          av[k][j] = ld_agent_u32(reinterpret_cast<const uint32_t*>(&A.mail.part[((rb + j) * NH + h) * DV + d0]));
+      for (int j = 0; j < BATCH; ++j) {
+        const int jl = kLongSplits ? max(min(j0 + j, nsp - 1), 0) : j;
+        load_words(rs, c0 * 2, (jl * NH + h0) * DV * 2, av[j]);
       }
-    }
+    };
+    const auto add = [&](int j0) {
+#pragma unroll
+      for (int j = 0; j < BATCH; ++j) {
+        const float w = Q.w[hh][j0 + j];
+        if (w > 0.f)
+#pragma unroll
+          for (int i = 0; i < CPT / 2; ++i) {
+            o[2 * i] += w * bf16_lo(av[j][i]);
+            o[2 * i + 1] += w * bf16_hi(av[j][i]);
+          }
+      }
+    };
+    if (mine) load(0);
     __syncthreads();
     if (mine) {
-#pragma unroll
-      for (int k = 0; k < IPT; ++k) {
-        const int it = tid + AT * k, hh = it / (DV / 2), h = h0 + hh, d0 = (it % (DV / 2)) * 2;
-        float o[2] = {0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < NSP; ++j) {
-          const float w = Q.w[hh][j];
-          if (w > 0.f) {
-            o[0] += w * bf16_lo(av[k][j]);
-            o[1] += w * bf16_hi(av[k][j]);
-          }
+      add(0);
+      if (kLongSplits)
+#pragma unroll 1
+        for (int j0 = BATCH; j0 < nsp; j0 += BATCH) {
+          load(j0);
+          add(j0);
         }
-        const float den = Q.den[hh];
-        const float inv = den > 0.f ? 1.0f / den : 0.f;
-        uint32_t* po = reinterpret_cast<uint32_t*>(A.out + ((size_t)s * NH + h) * DV + d0);
-        const uint32_t ov = pack_bf16x2(o[0] * inv, o[1] * inv);
+      const float den = Q.den[hh];
+      const float inv = den > 0.f ? 1.0f / den : 0.f;
+      uint32_t* po = reinterpret_cast<uint32_t*>(A.out + ((size_t)s * NH + h0) * DV + c0);
+#pragma unroll
+      for (int i = 0; i < CPT / 2; ++i) {
+        const uint32_t ov = pack_bf16x2(o[2 * i] * inv, o[2 * i + 1] * inv);
         if (A.publish_out) {  // read in this launch: a device-coherent store, complete before the done word
-          __hip_atomic_store(po, ov, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(po + i, ov, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
-          *po = ov;
+          po[i] = ov;
         }
       }
       if (A.publish_out) __builtin_amdgcn_s_waitcnt(0);

@@ -152,6 +152,25 @@ def test_attn_score_runs(rt, gpu_device, rows):
     assert torch.equal(out, rt.forward(step, caches))
 
 
+@pytest.mark.parametrize("rows,full", [(17, True), (17, False), (29, False), (33, True), (43, True), (64, True), (64, False)])
+def test_attn_split_plan(rt, gpu_device, rows, full):
+    """A wide step's selected tokens are shared out over at most 256 splits: one to eight
+    64-token sub-tiles each, fewer for short rows, none for an empty one (whose output is
+    zero); rows around a sub-tile's edges against the oracle."""
+    lens = [1, 63, 64, 65, 2047, 2049, 128, 129, 700, 1999, 5000]
+    ctx = [2048 + 37 * i for i in range(rows)] if full else [lens[(4 * i + i // 11) % 11] for i in range(rows)]
+    out, _, _ = _check(rt, ctx, 80 + rows, gpu_device)
+    step, caches = workloads.attn_case(ctx, gpu_device, seed=80 + rows)
+    step.seq_lens[rows // 2] = 0  # the other rows may take other splits: the same values but for rounding
+    got = rt.forward(step, caches)
+    torch.cuda.synchronize()
+    rt.check_errors()
+    assert bool((got[rows // 2] == 0).all())
+    keep = [s for s in range(rows) if s != rows // 2]
+    a, b = got[keep].float(), out[keep].float()
+    assert bool(((a - b).abs() <= OUT_MAX_ABS + OUT_REL * b.abs()).all()) and ((a - b).norm() / b.norm()).item() <= OUT_REL
+
+
 @pytest.mark.parametrize("period", [0, 1, 6])
 def test_attn_rows_of_one_member(rt, gpu_device, period):
     """Wide steps whose rows fit one top-k member (at most 8192 keys) beside rows that take
