@@ -558,7 +558,10 @@ class Step {
     L.red[1][wave][lane] = au;
     __syncthreads();
     if (tid < 256) {
-      const int l = tid % WAVE, i = tid / WAVE;
+      // a lane's four channels in neighbouring lanes: 32 contiguous bytes a row and store
+      // instruction (a wave a channel stored 8 bytes every 32; the down tasks' words go out
+      // in pairs for the same reason: 8 rows 92.9 -> 92.0 us, the layer 154.6 -> 152.6)
+      const int l = tid / 4, i = tid % 4;
       float gs = 0.f, us = 0.f;
 #pragma unroll
       for (int w = 0; w < FW; ++w) {
@@ -666,13 +669,15 @@ class Step {
     __syncthreads();
     if (!odd) acc[3] += L.red[0][wv + 1][lane];
     if ((mask >> r) & 1u) {
+      const __amdgpu_buffer_rsrc_t rs = coherent_rsrc(A.mail.ypart + (size_t)d * MAX_ROWS * H, MAX_ROWS * H * 8);
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
         if (odd && a == 0) continue;  // wave-uniform
+        const int at = (r * H + (rt0 + a + 3 * odd) * 16 + 4 * g) * 8;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int h = (rt0 + a + 3 * odd) * 16 + 4 * g + i;
-          mb_putf(&A.mail.ypart[((size_t)d * MAX_ROWS + r) * H + h], acc[a][i], gd.tag);
+        for (int i = 0; i < 4; i += 2) {
+          mb_put2f(rs, at + 8 * i, acc[a][i], acc[a][i + 1], gd.tag);
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
     }

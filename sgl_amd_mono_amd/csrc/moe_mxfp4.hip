@@ -581,12 +581,11 @@ class Step {
     }
     const int s = lane % 16;
     if ((mask >> s) & 1u) {
+      const __amdgpu_buffer_rsrc_t rs = coherent_rsrc(A.mail.mid + (size_t)d * MAX_ROWS * I, MAX_ROWS * I * 8);
+      const int at = (s * I + c * 16 + 4 * (lane / 16)) * 8;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int ch = c * 16 + 4 * (lane / 16) + i;
-        // mid is staged as bf16 (glm53/gfx950/kernel.py:5111-5117)
-        mb_putf(&A.mail.mid[((size_t)d * MAX_ROWS + s) * I + ch], bf16_round(silu(gs[i]) * us[i]), gd.tag);
-      }
+      for (int i = 0; i < 4; i += 2)  // mid is staged as bf16 (glm53/gfx950/kernel.py:5111-5117)
+        mb_put2f(rs, at + 8 * i, bf16_round(silu(gs[i]) * us[i]), bf16_round(silu(gs[i + 1]) * us[i + 1]), gd.tag);
     }
     // the tile's done word, after its mid words: a hint for the down tasks' wait (their
     // poll of the tagged mid words stays the check)
@@ -643,13 +642,13 @@ class Step {
     const int d = j / DN_GROUPS, grp = j % DN_GROUPS;
     const uint32_t mask = L.plan.rowmask[d];
     if ((mask >> r) & 1u) {
+      const __amdgpu_buffer_rsrc_t rs = coherent_rsrc(A.mail.ypart + (size_t)d * MAX_ROWS * H, MAX_ROWS * H * 8);
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t) {
+        const int at = (r * H + grp * DN_ROWS + wave * 32 + t * 16 + 4 * g) * 8;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int h = grp * DN_ROWS + wave * 32 + t * 16 + 4 * g + i;
-          mb_putf(&A.mail.ypart[((size_t)d * MAX_ROWS + r) * H + h], acc[t][i], gd.tag);
-        }
+        for (int i = 0; i < 4; i += 2) mb_put2f(rs, at + 8 * i, acc[t][i], acc[t][i + 1], gd.tag);
+      }
     }
   }
 

@@ -134,6 +134,15 @@ MONO_DEV __amdgpu_buffer_rsrc_t coherent_rsrc(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, BUF_DWORD3);
 }
 
+// Two neighbouring tagged words as one 16-byte store (each still its own payload and tag,
+// polled as 8-byte words). Every write-through store goes to memory by itself, so a lane
+// that holds consecutive outputs stores them together: the MXFP4 MoE of 16 rows, whose
+// last outputs landed 6 us after the last down group, went from 56.6 to 51.1 us a launch.
+MONO_DEV void mb_put2f(__amdgpu_buffer_rsrc_t rs, int byte, float a, float b, uint32_t tag) {
+  const u32x4 v = {__float_as_uint(a), tag, __float_as_uint(b), tag};
+  __builtin_amdgcn_raw_buffer_store_b128(v, rs, byte, 0, SC1);
+}
+
 // A done word that many workgroups poll is put in DONE_REPLICAS copies 4 KB apart
 // (apart in the memory channels) and workgroup b polls copy b % DONE_REPLICAS, so no
 // single line takes every workgroup's polls. An array of n replicated done words takes
