@@ -587,9 +587,6 @@ class Step {
       for (int i = 0; i < 4; i += 2)  // mid is staged as bf16 (glm53/gfx950/kernel.py:5111-5117)
         mb_put2f(rs, at + 8 * i, bf16_round(silu(gs[i]) * us[i]), bf16_round(silu(gs[i + 1]) * us[i + 1]), gd.tag);
     }
-    // the tile's done word, after its mid words: a hint for the down tasks' wait (their
-    // poll of the tagged mid words stays the check)
-    if (lane == 0) mb_put(&A.mail.mtile[T], 0u, gd.tag);
   }
 
   // ---------------------------------------------------------------- down
@@ -603,13 +600,13 @@ class Step {
     const uint64_t* b0 = &A.mail.mid[((size_t)d0 * MAX_ROWS + s) * I + c0];
     const uint64_t* b1 = &A.mail.mid[((size_t)d1 * MAX_ROWS + s) * I + c0];
     constexpr uint32_t ALL = (1u << MPT) - 1u;
-    // first the slots' up tile done words (one a thread, the rest at the barrier): a
-    // waiting workgroup then spins on at most 2 NT words instead of every mid word
-    const uint64_t* tiles = &A.mail.mtile[(size_t)d0 * NT];
-    if (!hint_wait((d1 - d0 + 1) * NT, [tiles](int i) { return tiles + i; }, W_MID, gd)) return false;
+    // every spin sweeps all missing words: waiting first on a done word of each up tile cost
+    // one more round trip and won nothing back (1 row 18.8 -> 18.4 us a launch without it, 2
+    // rows 22.0 -> 21.7, 3 rows 25.1 -> 24.8, 4 to 16 rows within noise)
     uint32_t v[2 * MPT];
-    const bool ok = poll_words<2 * MPT>([b0, b1](int q) { return q < MPT ? b0 + q : b1 + (q - MPT); }, v,
-                                        (in0 ? ALL : 0u) | (in1 ? ALL << MPT : 0u), W_MID, gd);
+    const auto at = [b0, b1](int q) { return q < MPT ? b0 + q : b1 + (q - MPT); };
+    const bool ok = poll_words<2 * MPT, decltype(at), false, false>(at, v, (in0 ? ALL : 0u) | (in1 ? ALL << MPT : 0u),
+                                                                    W_MID, gd);
     if (!block_all(ok)) return false;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
