@@ -26,9 +26,10 @@
 //   plan     the distinct experts of the step; slot 0 is the shared expert (weight 1),
 //            slots 1.. the picked experts by ascending id
 //   tasks    one round-robin list over the workgroups:
-//            up     (slot, 16-channel tile; the shared expert's before the plan): FP8 x FP8 MFMA 16x16x128 with the 128x128
-//                   weight block scale x the activation block scale per 128-k, the 8
-//                   waves splitting K, SiLU(gate) * up -> mailbox mid
+//            up     (slot, 16-channel tile; the shared expert's are done before the plan):
+//                   FP8 x FP8 MFMA 16x16x128 with the 128x128 weight block scale x the
+//                   activation block scale per 128-k, the 8 waves splitting K,
+//                   SiLU(gate) * up -> mailbox mid
 //            down   (slot, 448 output rows): the slot's mid quantised per 128 to FP8 in
 //                   LDS (kernel.py:5118-5125), FP8 MFMA, x weight block scale x mid
 //                   block scale x route weight -> mailbox ypart
