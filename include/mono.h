@@ -220,7 +220,13 @@ typedef struct {
   int64_t* timeline;         /* optional i64 [tasks, 4] per task of the launch: start,
                                 inputs-ready and end s_memrealtime ticks (100 MHz), and
                                 workgroup << 8 | kind (the reference's timeline stamps,
-                                common/stamps.py:24-33) */
+                                common/stamps.py:24-33): rows x max_ctx / 1024 score tasks
+                                (padded to a multiple of a row's top-k members), rows x
+                                members (16, above 16 rows 4), rows x splits (32, above 16
+                                rows ceil(256 / rows)) and rows x merges (32, above 16 rows
+                                8, above 32 rows 4). A row of a task that the step does not
+                                have (a chunk past its row, a split that the plan leaves
+                                out) ends where it starts. */
 } mono_attn_args;
 
 int mono_attn_forward(mono_attn* attn, const mono_attn_args* args, void* stream);

@@ -82,7 +82,8 @@ class AttnRuntime(Runtime):
         index scores [rows, max_ctx] and the selected slots [rows, 2048]. ``timeline``
         (int64 [n_tasks(rows), 4]) receives each task's start, inputs-ready and end
         s_memrealtime ticks (100 MHz) and workgroup << 8 | kind (0 score, 1 top-k,
-        2 split, 3 merge)."""
+        2 split, 3 merge); a row of a task that this step does not have (a chunk past its
+        row, a split that the plan leaves out) ends where it starts."""
         args, out, dbg = self.args(step, caches, out, debug, timeline)
         _lib.check(_lib.lib().mono_attn_forward(self._h, C.byref(args), self._stream()))
         return (out, dbg) if debug else out

@@ -324,8 +324,11 @@ class Step {
       if (!ok) return false;
     }
     const int tlm = n_score() + n_topk + A.rows * splits_of(A.rows);
-    if (!kLongSplits) return merges<1>(at + n_split, tlm);
-    return merges_of(A.rows) == 8 ? merges<4>(at + n_split, tlm) : merges<8>(at + n_split, tlm);
+    const bool ok = !kLongSplits               ? merges<1>(at + n_split, tlm)
+                    : merges_of(A.rows) == 8 ? merges<4>(at + n_split, tlm)
+                                             : merges<8>(at + n_split, tlm);
+    if (A.timeline) stamp_idle(n_split);
+    return ok;
   }
 
  private:
@@ -394,6 +397,18 @@ class Step {
     }
   }
   MONO_DEV void mark_waited() { waited = now_ticks(); }
+  // The timeline rows that no task of this step has, as tasks that end where they start:
+  // chunks that are not scored (with the padding to whole teams) and splits past the plan.
+  MONO_DEV void stamp_idle(int n_split) {
+    waited = 0;
+    for (int T = block_index(); T < n_score(); T += G) {
+      const int s = T / CH;
+      if (s >= A.rows || T % CH >= live_chunks(row_len(s))) stamp(T, now_ticks(), 0);
+    }
+    if (kLongSplits)
+      for (int i = first_at_or_after(n_split); i < A.rows * splits_of(A.rows); i += G)
+        stamp(n_score() + n_topk() + i, now_ticks(), 2);
+  }
 
   // ---------------------------------------------------------------- score
   // The row's FP4 query in a wave's MFMA operands (64 heads x 128 dims: head tile ht =

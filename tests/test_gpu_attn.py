@@ -16,7 +16,7 @@ import torch
 
 from oracle import attention as oatt
 from sgl_amd_mono_amd import workloads
-from sgl_amd_mono_amd.attn import AttnRuntime
+from sgl_amd_mono_amd.attn import AttnRuntime, merges_of, splits_of
 
 pytestmark = pytest.mark.gpu
 
@@ -253,6 +253,32 @@ def test_attn_ties_take_lowest_positions(rt, gpu_device):
     for s in range(2):
         want = (pt[s, pos // 64].long() * 64 + pos % 64).to(torch.int32)
         assert torch.equal(dbg["topk"][s].cpu(), want)
+
+
+@pytest.mark.parametrize("rows,max_ctx", [(3, 1024), (8, 32768), (13, 32768), (20, 3072), (33, 32768), (64, 32768)])
+def test_attn_timeline_rows_all_written(gpu_device, rows, max_ctx):
+    """A launch writes every row of its timeline, those of the tasks that the step does
+    not have among them (chunks past a row or of a row that is not scored, the padding to
+    whole top-k teams, splits that the plan leaves out): no stale row is left."""
+    lens = [min(n, max_ctx) for n in ([700, 5000, 2049, 64, 20000, 2048] * 11)[:rows]]
+    step, caches = workloads.attn_case(lens, gpu_device, seed=14, max_ctx=max_ctx)
+    r = AttnRuntime(rows, max_ctx, device=gpu_device)
+    try:
+        tl = torch.full((r.n_tasks(rows), 4), -1, dtype=torch.int64, device=gpu_device)
+        out = r.forward(step, caches, timeline=tl)
+        plain = r.forward(step, caches)
+        torch.cuda.synchronize()
+        r.check_errors()
+    finally:
+        r.close()
+    tl = tl.cpu()
+    team = 16 if rows <= 16 else 4
+    n = [-(-rows * (max_ctx // 1024) // team) * team, rows * team, rows * splits_of(rows), rows * merges_of(rows)]
+    kinds = torch.repeat_interleave(torch.arange(4), torch.tensor(n))
+    assert torch.equal(tl[:, 3] & 255, kinds), int((tl[:, 3] & 255 != kinds).sum())
+    assert bool((tl[:, 0] > 0).all() and (tl[:, 2] >= tl[:, 0]).all() and (tl[:, 1] >= 0).all())
+    assert bool((tl[:, 3] >> 8 < torch.cuda.get_device_properties(gpu_device).multi_processor_count).all())
+    assert torch.equal(out, plain)
 
 
 def test_attn_repeat_is_bitwise(rt, gpu_device):
