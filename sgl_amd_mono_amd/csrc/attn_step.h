@@ -56,12 +56,6 @@ constexpr int TMK = TEAM_LONG;  // members of a row's top-k team in this launch
 constexpr bool kLongSplits = false;
 constexpr int TMK = TEAM;
 #endif
-// the launch may run the front too (a whole layer): the attention waits for its outputs
-#ifdef MONO_ATTN_FRONT
-constexpr bool kFront = true;
-#else
-constexpr bool kFront = false;
-#endif
 
 constexpr int AT = 512;
 constexpr int AW = AT / WAVE;
@@ -193,9 +187,12 @@ struct Args {
   float scale;
   // the front of the layer ran earlier in this launch: its replicated done words
   // (proj::Mail::fdone: FD_B + s row s's index key and head weights, FD_E + 8 s + j its
-  // index query, FD_D + h head h of q), awaited at wait sites fsite and fsite + 1
+  // index query, FD_D + h head h of q), awaited at wait sites fsite and fsite + 1; only a
+  // build with MONO_ATTN_FRONT has the waits, so no other build can name done words
+#ifdef MONO_ATTN_FRONT
   const uint64_t* fdone;
   int fsite;
+#endif
   bool publish_out;  // a later stage of the launch reads `out`: each merge puts a done word
   // the row histograms: 1, two copies by launch parity (each launch clears its
   // successor's copy, the guard's flip words); 0, one copy that the launch's caller
@@ -586,12 +583,21 @@ class Step {
   // own new key and, for the rows of a verify chain, those of the chain's earlier rows;
   // a wave past the row reads the row's last page).
   MONO_DEV bool fresh(int k0, int n) const { return front_here() && k0 + KEYS_WAVE > n - A.rows; }  // wave-uniform
-  MONO_DEV bool front_here() const { return kFront && A.fdone; }
+  MONO_DEV bool front_here() const { return front_done() != nullptr; }
+  // the done words of the front of this launch (null, at compile time: it runs no front)
+  // and the wait site of its first outputs
+#ifdef MONO_ATTN_FRONT
+  MONO_DEV const uint64_t* front_done() const { return A.fdone; }
+  MONO_DEV int front_site() const { return A.fsite; }
+#else
+  MONO_DEV const uint64_t* front_done() const { return nullptr; }
+  MONO_DEV int front_site() const { return 0; }
+#endif
   MONO_DEV bool await_front() {
-    const uint64_t* fd = done_copy(A.fdone);
+    const uint64_t* fd = done_copy(front_done());
     const int nr = A.rows;
     return hint_wait(nr * (1 + IH / 8), [fd, nr](int i) { return fd + (i < nr ? proj::FD_B + i : proj::FD_E + i - nr); },
-                     A.fsite, gd);
+                     front_site(), gd);
   }
 
   // This workgroup's share of the scores, and `base` for the tasks after them.
@@ -695,8 +701,6 @@ class Step {
       if (awaited) {
         key_load(z, ka, pages_of(z, 0));
         key_load(z, kb, pages_of(z, 1));
-        if (!planned) plan_splits();
-        planned = true;
       } else {
         const auto fresh_at = [&](int j) {
           const int sj = row_at(i0 + min(j, m - 1));
@@ -712,6 +716,8 @@ class Step {
         if (fb) key_load(z, kb, pages_of(z, 1));
         __syncthreads();
       }
+      if (!planned) plan_splits();
+      planned = true;
       Query q;
       int n = 0, c = -1, c0 = 0;
       const auto turn = [&](Keys& k, int j) {  // chunk j of the piece
@@ -1224,9 +1230,9 @@ class Step {
     if (front_here() && !q_ready) {
       // every head of q from the front of this launch, and every row's cache row (a row that
       // selects all its keys waits for no scores, which would follow them)
-      const uint64_t* fd = done_copy(A.fdone);
+      const uint64_t* fd = done_copy(front_done());
       if (!hint_wait(NH + A.rows, [fd](int i) { return fd + (i < NH ? proj::FD_D + i : proj::FD_B + i - NH); },
-                     A.fsite + 1, gd))
+                     front_site() + 1, gd))
         return false;
       q_ready = true;
     }
@@ -1572,8 +1578,10 @@ void fill_args(Args& a, const AttnArgs& g, const Mail& mail, const GuardArgs& gu
   a.scale = g.softmax_scale;
   a.publish_out = false;
   a.rowh_flip = 1;
+#ifdef MONO_ATTN_FRONT
   a.fdone = nullptr;
   a.fsite = 0;
+#endif
   a.mail = mail;
   a.guard = guard;
 }
