@@ -152,6 +152,25 @@ def test_attn_score_runs(rt, gpu_device, rows):
     assert torch.equal(out, rt.forward(step, caches))
 
 
+@pytest.mark.parametrize("rows", [9, 13, 16])
+def test_attn_empty_rows_of_score_runs(rt, gpu_device, rows):
+    """Empty rows (length 0) in steps of up to 16 rows whose scored chunks run in shares: the
+    first, one in the middle, the last and then every one. Their output is zero and, each row
+    keeping its splits, the others' stay bit for bit."""
+    ctx = [[4096, 2049, 700, 9000, 2048][i % 5] for i in range(rows)]
+    step, caches = workloads.attn_case(ctx, gpu_device, seed=90 + rows)
+    want = rt.forward(step, caches).clone()
+    step.seq_lens[[0, rows // 2, rows - 1]] = 0
+    got = rt.forward(step, caches).clone()
+    step.seq_lens.zero_()
+    none = rt.forward(step, caches)
+    torch.cuda.synchronize()
+    rt.check_errors()
+    for s in range(rows):
+        assert torch.equal(got[s], want[s]) if s not in (0, rows // 2, rows - 1) else bool((got[s] == 0).all()), s
+    assert bool((none == 0).all())
+
+
 @pytest.mark.parametrize("rows,full", [(17, True), (17, False), (29, False), (33, True), (43, True), (64, True), (64, False)])
 def test_attn_split_plan(rt, gpu_device, rows, full):
     """A wide step's selected tokens are shared out over at most 256 splits: one to eight

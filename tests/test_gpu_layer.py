@@ -218,6 +218,39 @@ def test_layer_launch_modes_agree_bitwise(gpu_device, rows):
                 assert torch.equal(it[k], ir[k]), (mode, k)
 
 
+@pytest.mark.parametrize("rows,lens", [
+    (12, [30000, 1, 2048, 2049, 9000, 64, 3072, 3073, 20000, 2050, 700, 32768]),
+    (16, [2500] * 8 + [1, 64, 2048, 30000, 2047, 65, 1024, 5000]),
+    (16, [1, 2048, 64, 700, 2047, 1023, 1024, 65] * 2),
+    (3, [2048, 700, 1]),
+])
+def test_layer_launch_modes_without_debug_outputs(gpu_device, rows, lens):
+    """As served: no debug outputs asked for, so rows of at most 2048 keys are not scored and
+    their splits take every key without a selection. The fused launches at 32768 keys (above
+    8 rows the scored chunks run in shares over the workgroups) give bit for bit the split
+    launches' rows, and the same as with debug outputs, where every row is scored."""
+    ctx = 32768
+    cos, sin = workloads.rope_tables(ctx, gpu_device)
+    print(f"[modes, plain] rows={rows}", flush=True)
+    w = LayerWeights(proj=workloads.proj_weights(gpu_device, seed=35),
+                     moe=workloads.fp8_moe_weights(FP8_MOE, gpu_device, seed=36))
+    x = workloads.rows_bf16(rows, ol.HIDDEN, gpu_device, seed=38)
+    got = {}
+    for mode in ("layer", "attn_back", "split"):
+        step, caches = workloads.attn_case(lens, gpu_device, seed=37, max_ctx=ctx)
+        rt = LayerRuntime(rows, ctx, gpu_device, mode=mode)
+        try:
+            args = (x, step.seq_lens, step.page_table, caches, w, cos, sin)
+            got[mode] = [rt.forward(*args).clone() for _ in range(2)] + [rt.forward(*args, keep=True)[0].clone()]
+            torch.cuda.synchronize()
+            rt.check_errors()
+        finally:
+            rt.close()
+    for mode, outs in got.items():
+        for k, o in enumerate(outs):
+            assert torch.equal(o, got["split"][0]), (mode, k)
+
+
 @pytest.mark.parametrize("site,what", [(10, "attention block output rows"), (11, "front: stage-A partial sums"),
                                        (17, "front index query and keys"), (18, "front q")])
 def test_layer_launch_fail_stop(gpu_device, site, what):

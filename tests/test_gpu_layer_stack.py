@@ -24,12 +24,12 @@ def _weights(dev, n, seed0):
     return [sets[l % 2] for l in range(n)]
 
 
-def _case(dev, n, rows, seed):
+def _case(dev, n, rows, seed, ctx=CTX, lens=None):
     """Each layer's own caches (one attn_case a layer) and the step's input rows."""
-    lens = ([CTX, 1500, 65, 2049, 4000, 64, 7000, 300] * 2)[:rows]
+    lens = (lens or [CTX, 1500, 65, 2049, 4000, 64, 7000, 300] * 2)[:rows]
     steps, caches = [], []
     for l in range(n):
-        st, c = workloads.attn_case(lens, dev, seed=seed + l, max_ctx=CTX)
+        st, c = workloads.attn_case(lens, dev, seed=seed + l, max_ctx=ctx)
         steps.append(st)
         caches.append(c)
     x = workloads.rows_bf16(rows, ol.HIDDEN, dev, seed=seed + 100)
@@ -94,6 +94,41 @@ def test_stack_equals_one_launch_a_layer(gpu_device, rows, n):
         words = rt.handle.error_words()
         ordinal = (words[_lib.G_TICKET] & 0xFFFFFFFF) | (words[_lib.G_TICKET + 1] & 0xFFFFFFFF) << 32
         assert ordinal == 3 * (n + n % 2) + 1, ordinal
+    finally:
+        rt.close()
+        ref.close()
+
+
+@pytest.mark.parametrize("rows", [12, 14, 16])
+@pytest.mark.parametrize("short", [False, True])
+def test_stack_of_wide_steps_at_long_contexts(gpu_device, rows, short):
+    """Steps whose chunks of max_ctx outnumber the workgroups, so that the scored chunks run
+    in shares inside the multi-layer launch: up to 14 rows stage D follows the top-k members'
+    place in that list, at 16 it stays in the front. Rows around the selection's edge beside
+    long ones, or (short) no scored row at all, whose index queries nobody waits for. Two
+    stacked steps equal one launch a layer bit for bit (a histogram left uncleared by the
+    first would change the second's selections)."""
+    ctx, n = 32768, 3
+    lens = [1, 2048, 64, 700, 2047, 1023, 1024, 65] * 2 if short else [
+        30000, 1, 2048, 2049, 9000, 64, 3072, 3073, 20000, 2050, 700, 32768, 5000, 4096, 2047, 12000]
+    print(f"[stack] rows={rows} ctx={ctx} short={short}", flush=True)
+    cos, sin = workloads.rope_tables(ctx, gpu_device)
+    ws = _weights(gpu_device, n, 320)
+    steps, caches, x = _case(gpu_device, n, rows, 330 + rows, ctx, lens)
+    ref_caches = [_clone(c) for c in caches]
+    ref = LayerRuntime(rows, ctx, gpu_device)
+    rt = LayerRuntime(rows, ctx, gpu_device, max_layers=n)
+    try:
+        want = _one_by_one(ref, x, steps, ref_caches, ws, cos, sin)
+        for k in range(2):
+            got = _stack(rt, x, steps, caches, ws, cos, sin)
+            torch.cuda.synchronize()
+            rt.check_errors()
+            ref.check_errors()
+            _same(got, want, f"stacked step {k}")
+        for c, r in zip(caches, ref_caches):
+            for f in ("kv", "ikv", "iks", "kv_scale"):
+                assert torch.equal(getattr(c, f), getattr(r, f)), f
     finally:
         rt.close()
         ref.close()
