@@ -901,7 +901,7 @@ class Step {
       uint32_t v[TMK];
       const uint64_t* col = hb + tid;
       const auto at = [col](int j) { return col + j * HW; };
-      ok = poll_words<TMK, decltype(at), false, false>(at, v, (1u << TMK) - 1u, W_TEAM, gd);
+      ok = poll_words<TMK, decltype(at), false>(at, v, (1u << TMK) - 1u, W_TEAM, gd);
       uint32_t t = 0, p = 0;  // two 16-bit sums side by side (at most TMK KPM keys)
 #pragma unroll
       for (int j = 0; j < TMK; ++j) {

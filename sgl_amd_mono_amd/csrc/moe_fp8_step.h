@@ -81,6 +81,7 @@ static_assert(UP_KBW * 2 == 14 && DN_PAIR * IB == 2 * 14 && H % DN_ROWS == 0, "1
 static_assert(IB == 4 && DN_PAIR == 7, "a wave pair's row tiles: 3 whole and half of one each");
 static_assert(I == 8 * WAVE && MAX_ROWS <= 2 * FW, "a down task's wave reads one or two mid rows, 8 channels a lane");
 static_assert(MAX_ROWS * FIN_ROWS <= FT, "a final task's thread owns one (row, output)");
+static_assert(H % 2 == 0, "pairs of tagged words at 16-byte addresses (mb_put2f)");
 
 // wait sites (guard error word = site + 1), offset by the Step's site0 in a fused
 // launch; W_A: the attention block's output rows (fused launch only)
@@ -724,8 +725,7 @@ class Step {
       // every spin sweeps all missing words (no probe): the finals wait at the tail, when
       // the weight streams are over, and a probe's extra round trip is what costs there
       const auto at = [base, slots](int k) { return base + (size_t)slots[k] * MAX_ROWS * H; };
-      ok = poll_words<NSLOT, decltype(at), false, false>(at, v,
-                             (1u << NSLOT) - 1u, site0 + W_YPART, gd);
+      ok = poll_words<NSLOT, decltype(at), false>(at, v, (1u << NSLOT) - 1u, site0 + W_YPART, gd);
       if (ok) {
         float y = 0.f;
 #pragma unroll

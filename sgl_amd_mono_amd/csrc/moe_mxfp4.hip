@@ -71,6 +71,7 @@ static_assert(HS % FW == 0 && I % 128 == 0 && I % MPT == 0 && MPT % 2 == 0, "til
 static_assert(2 * UP_SW == NW && 2 * IS == NW && DN_ROWS == FW * 32, "six 16-byte weight loads a lane a task");
 static_assert(MAX_ROWS <= 2 * FW && MAX_ROWS == 16, "two rows a wave to route; an MFMA column a row");
 static_assert(MAX_ROWS * FIN_ROWS <= FT, "a final task's thread owns one (row, output)");
+static_assert(I % 2 == 0 && H % 2 == 0, "pairs of tagged words at 16-byte addresses (mb_put2f)");
 // a workgroup's block of down groups holds at most ceil(slots * DN_GROUPS / grid) groups
 // and spans at most two slots while that is at most DN_GROUPS + 1: grids of MIN_GRID
 // workgroups and more (the launcher refuses smaller ones)
@@ -605,8 +606,8 @@ class Step {
     // rows 22.0 -> 21.7, 3 rows 25.1 -> 24.8, 4 to 16 rows within noise)
     uint32_t v[2 * MPT];
     const auto at = [b0, b1](int q) { return q < MPT ? b0 + q : b1 + (q - MPT); };
-    const bool ok = poll_words<2 * MPT, decltype(at), false, false>(at, v, (in0 ? ALL : 0u) | (in1 ? ALL << MPT : 0u),
-                                                                    W_MID, gd);
+    const bool ok = poll_words<2 * MPT, decltype(at), false>(at, v, (in0 ? ALL : 0u) | (in1 ? ALL << MPT : 0u),
+                                                             W_MID, gd);
     if (!block_all(ok)) return false;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -661,8 +662,7 @@ class Step {
       // every spin sweeps all missing words (no probe): the finals wait at the tail, when
       // the weight streams are over, and a probe's extra round trip is what costs there
       const auto at = [base, slots](int k) { return base + (size_t)slots[k] * MAX_ROWS * H; };
-      ok = poll_words<NSLOT, decltype(at), false, false>(at, v,
-                             (1u << NSLOT) - 1u, W_YPART, gd);
+      ok = poll_words<NSLOT, decltype(at), false>(at, v, (1u << NSLOT) - 1u, W_YPART, gd);
       if (ok) {
         float y = 0.f;
 #pragma unroll

@@ -1,10 +1,18 @@
 // Inter-workgroup hand-off inside one persistent launch: tagged mailbox words and the
 // guard that bounds every wait.
 //
-// A mailbox word is 64 bits: the payload (an f32 or i32's bits) in the low half and
-// the launch's tag in the high half, written by one agent-scope relaxed atomic store
-// (global_store_dwordx2 sc1) and read by agent-scope relaxed atomic loads
-// (global_load_dwordx2 sc1). The tag makes every word self-validating, so a producer
+// A mailbox word is 64 bits at an 8-byte aligned address: the payload (an f32 or i32's
+// bits) in the low half and the launch's tag in the high half, read by agent-scope
+// relaxed atomic loads (global_load_dwordx2 sc1) and written whole by one device-coherent
+// store instruction, in one of three forms:
+//   mb_put     one word by an agent-scope relaxed atomic store (global_store_dwordx2 sc1)
+//   buffer     one word by an 8-byte buffer store (buffer_store_dwordx2 sc1: the top-k's
+//              selected slots, where out-of-range words are dropped)
+//   mb_put2f   two neighbouring words by a 16-byte buffer store (buffer_store_dwordx4 sc1)
+//              at a 16-byte aligned address
+// What all of them rest on: an aligned 8-byte half of one lane's store becomes visible
+// as a whole, payload and tag together (the two words of a 16-byte store may be seen one
+// after the other). The tag makes every word self-validating, so a producer
 // needs no release fence and a consumer no acquire fence: on gfx950 those are an L2
 // writeback / invalidate of the XCD, which costs far more than the hand-off. This is
 // the reference's tagged (value, tag) pair (sgl_amd_mono/common/sync.py:30-207,
@@ -104,10 +112,6 @@ MONO_DEV void mb_putf(uint64_t* p, float v, uint32_t tag) { mb_put(p, __float_as
 MONO_DEV uint64_t mb_load(const uint64_t* p) {
   return __hip_atomic_load(const_cast<uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// A plain (L2-cacheable) load of a mailbox word. Only a first pass after a hint wait
-// uses it: a line cached before its producer wrote it returns an old tag, and that word
-// is then polled with agent-scope loads, so a stale copy is never taken for data.
-MONO_DEV uint64_t mb_load_cached(const uint64_t* p) { return *p; }
 MONO_DEV uint32_t ld_agent_u32(const uint32_t* p) {
   return __hip_atomic_load(const_cast<uint32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -135,7 +139,8 @@ MONO_DEV __amdgpu_buffer_rsrc_t coherent_rsrc(const void* p, uint32_t bytes) {
 }
 
 // Two neighbouring tagged words as one 16-byte store (each still its own payload and tag,
-// polled as 8-byte words). Every write-through store goes to memory by itself, so a lane
+// polled as 8-byte words), at byte `byte` (a multiple of 16) of a resource whose base is
+// 16-byte aligned. Every write-through store goes to memory by itself, so a lane
 // that holds consecutive outputs stores them together: the MXFP4 MoE of 16 rows, whose
 // last outputs landed 6 us after the last down group, went from 56.6 to 51.1 us a launch.
 MONO_DEV void mb_put2f(__amdgpu_buffer_rsrc_t rs, int byte, float a, float b, uint32_t tag) {
@@ -218,29 +223,15 @@ struct Guard {
 // waiting workgroup then costs one load a thread a spin, not one a word, so early
 // waiters do not flood the memory system the producers are streaming through.
 //
-// CACHED_FIRST: the first pass uses plain cacheable loads (after a hint wait has seen the
-// producers finish, so many workgroups reading one broadcast payload share the L2 of
-// their XCD instead of each fetching it from memory).
-// PROBE = false: every spin sweeps all missing words (for small exchanges between a few
-// workgroups, where a probe's extra round trip is the cost that matters).
-template <int N, class At, bool CACHED_FIRST = false, bool PROBE = true>
+// PROBE = false: every spin sweeps all missing words, where a probe's extra round trip
+// costs more than the loads: the top-k team's exchange of a few words, the MoEs' final
+// tasks (at the tail, when the weight streams are over) and the MXFP4 MoE's mids (the
+// streams still run; moe_mxfp4.hip stage_mids has the figures).
+template <int N, class At, bool PROBE = true>
 MONO_DEV bool poll_words(At at, uint32_t (&v)[N], uint32_t pending, int site, const Guard& g) {
   if (pending && site == g.fault) {  // host-forced fault: the wait fails at once
     g.fail(site);
     return false;
-  }
-  if (CACHED_FIRST) {
-    uint64_t w[N];
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-      if ((pending >> j) & 1u) w[j] = mb_load_cached(at(j));
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-      if (((pending >> j) & 1u) && (uint32_t)(w[j] >> 32) == g.tag) {
-        v[j] = (uint32_t)w[j];
-        pending &= ~(1u << j);
-      }
-    if (!pending) return true;
   }
   const auto sweep = [&]() {
     uint64_t w[N];
@@ -294,11 +285,10 @@ MONO_DEV bool poll_word(const uint64_t* p, uint32_t& v, int site, const Guard& g
   return ok;
 }
 
-// Wait until each of n hint words carries the tag: thread i < n polls at(i), one word
-// that producer i of the awaited data writes with (or after) the rest of its share,
-// while the other threads wait at the barrier. The full poll that follows then mostly
-// finds every word in place on its first pass; meanwhile a waiting workgroup costs n
-// loads a spin instead of one a payload word. Workgroup-uniform result.
+// Wait until each of n done words carries the tag: thread i polls at(i), at(i + threads)
+// .., words that the producers of the awaited data put once their shares are stored, while
+// the other threads wait at the barrier. A waiting workgroup then costs n loads a spin, and
+// untagged data may be read after it. Workgroup-uniform result.
 template <class At>
 MONO_DEV bool hint_wait(int n, At at, int site, const Guard& g) {
   bool ok = true;
