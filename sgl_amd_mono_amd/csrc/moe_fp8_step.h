@@ -169,17 +169,21 @@ class Step {
       refused = true;
       return false;
     }
-    // the first router task's weights (or the workgroup's shared-expert tile's) and the route's biases go
-    // out before anything waits
+    // the first router task's weights (without one: those of the workgroup's tile of the
+    // shared expert, if it has one) and the route's biases go out before anything waits
     const int n_rt = RT_EG * ((S + RT_S - 1) / RT_S);
     int t = block_index();
     const f32x4 bias4 = *reinterpret_cast<const f32x4*>(A.bias + 4 * lane);
     const float bias[4] = {bias4[0], bias4[1], bias4[2], bias4[3]};
-    // The shared expert's up tiles need no routing: the last workgroups (the first to have
-    // no router task) take one each before the plan, its weights on their way while the
-    // router tasks run. As the first tiles of the list they gave 32 workgroups a second
-    // tile after the plan where everyone else had one (1 row: 34.9 -> 33.9 us; four stacked
-    // layers of 8 rows: 152.4 -> 150.6 us a layer).
+    // The shared expert's up tiles need no routing: the last workgroups take one each before
+    // the plan. Up to 6 rows these are workgroups without a router task (64 for every two
+    // rows), and the tiles' weights are on their way while the router tasks run. From 7 rows
+    // on every workgroup of 256 has a router task: there the 32 issue their tile's 229 KB
+    // between that task and the gather, whose words then return behind it (the MoE's
+    // prologue in an 8-row layer 17.5 -> 18.2 us), and the gain is the stream's alone. As the
+    // first tiles of the list they gave 32 workgroups a second tile after the plan where
+    // everyone else had one (1 row: 34.9 -> 33.9 us; four stacked layers of 8 rows: 152.4 ->
+    // 150.6 us a layer).
     const int e0 = G - 1 - t;
     if (t < n_rt) {
       u32x4 wr[RT_E][2], gr[2];
