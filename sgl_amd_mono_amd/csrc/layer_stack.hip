@@ -41,7 +41,17 @@ MONO_DEV void clear_words(uint32_t* p, uint32_t n) {
 // starts in a workgroup once that workgroup is done with the layer before; it waits only
 // on its own phases and on the layer before's final tasks (the done words of its input
 // rows), and it clears the layer before's row histograms, whose readers the layer
-// before's MoE plan has waited for. Each layer's buffers that a later layer rewrites
+// before's MoE plan has waited for.
+//
+// A few words of a layer have no reader in it: its index queries' done words when no row
+// is scored (all at most TOPK keys), and the scores of such rows in a launch with debug
+// outputs. What keeps the workgroup that writes them from falling behind into the next
+// layer, where the same mailboxes are written again, is its back task: the back's N_TASKS
+// tasks are dealt round-robin, so in a grid of at most as many workgroups each has one,
+// which follows its share of the front and the scores, and no final task of the layer ends
+// before every back task has. stack_forward refuses a larger grid.
+//
+// Each layer's buffers that a later layer rewrites
 // differ from every other layer's (the table's packer checks it), so no cache holds a
 // line a later layer of the launch rewrites.
 __global__ __launch_bounds__(512, 1) void k_layers(StackArgs args) {
@@ -89,7 +99,8 @@ hipError_t stack_fill(void* entry, const StackLayer& sl, const mono_proj_weights
 
 hipError_t stack_forward(const void* table, int n_layers, uint32_t rowh_words, const GuardArgs& guard, int grid,
                          hipStream_t st) {
-  if (n_layers < 1 || grid < 1 || !table) return hipErrorInvalidConfiguration;
+  // (a back task a workgroup: see k_layers)
+  if (n_layers < 1 || grid < 1 || grid > proj::Back::N_TASKS || !table) return hipErrorInvalidConfiguration;
   StackArgs a;
   a.table = (const __attribute__((address_space(4))) LayerArgs*)table;
   a.n_layers = n_layers;
