@@ -101,8 +101,9 @@ def test_attn_48_rows_mixed_contexts(rt, gpu_device):
 
 
 def test_attn_24_rows_long_splits(rt, gpu_device):
-    """24 rows take 8 splits a row of 256 selected tokens (four sub-tiles each) and merges
-    of 4 heads: the same selection and, within the bound, the same output."""
+    """24 rows of 1 to 32768 keys: splits of several sub-tiles shared out over the workgroups
+    (a full row's are 8 of 256 selected tokens, or more and shorter ones where other rows are
+    short) and merges of 4 heads, against the oracle."""
     g = torch.Generator().manual_seed(4)
     ctx = torch.randint(1, 32768, (24,), generator=g).tolist()
     ctx[0], ctx[1], ctx[2], ctx[3] = 32768, 2048, 2049, 300
@@ -110,15 +111,16 @@ def test_attn_24_rows_long_splits(rt, gpu_device):
 
 
 def test_attn_48_rows_full_contexts(rt, gpu_device):
-    """BASELINE config 3 at its largest size: 48 rows of (nearly) 32768 keys each (5 splits
-    a row of 6 or 7 sub-tiles, merges of 8 heads)."""
+    """BASELINE config 3 at its largest size: 48 rows of (nearly) 32768 keys each: 5 splits
+    a row of 6 or 7 sub-tiles (seven is the least with which 48 rows fit 256 splits), merges
+    of 8 heads."""
     ctx = [32768] * 44 + [32767, 32704, 30001, 16385]
     _check(rt, ctx, 7, gpu_device)
 
 
 def test_attn_56_rows_wide_launch(rt, gpu_device):
-    """Above 48 rows the launch takes 4 even splits a row (its own kernel build): the same
-    selection and, within the bound, the same output."""
+    """56 rows of 1 to 32768 keys: a step whose full rows would take 4 splits of 8 sub-tiles,
+    the most that a split holds, beside short rows that take fewer, against the oracle."""
     g = torch.Generator().manual_seed(11)
     ctx = torch.randint(1, 32768, (56,), generator=g).tolist()
     ctx[0], ctx[1], ctx[2], ctx[3] = 32768, 2048, 2049, 300
