@@ -78,7 +78,8 @@ class AttnRuntime(Runtime):
 
     def forward(self, step: AttnStep, caches: AttnCaches, out: torch.Tensor | None = None,
                 debug: bool = False, timeline: torch.Tensor | None = None):
-        """o_lat [rows, 32, 512] bf16 for one decode step. ``debug`` also returns the
+        """o_lat [rows, 32, 512] bf16 for one decode step (above 16 rows a row's last bits
+        depend on the other rows' lengths, which decide how its tokens are split). ``debug`` also returns the
         index scores [rows, max_ctx] and the selected slots [rows, 2048]. ``timeline``
         (int64 [n_tasks(rows), 4]) receives each task's start, inputs-ready and end
         s_memrealtime ticks (100 MHz) and workgroup << 8 | kind (0 score, 1 top-k,

@@ -346,7 +346,8 @@ class Step {
   // fixed count a row (8 to 32 rows, 5 to 48, 4 above) gave 33 rows splits of 7 sub-tiles
   // where 5 fit, 17 rows 4 where 3 fit, and a short row's first splits as much as they held
   // (33 rows of 1500-12000 keys: 47.9 -> 42.6 us a launch). Taken while the first keys are
-  // on their way.
+  // on their way. It takes in every row's length: a row's cuts, and with them its last bits,
+  // depend on the step's other rows (its error does not: 0.0026 of the exact values either way).
   MONO_DEV void plan_splits() {
     const int nst = sub_tiles(row_n);
     const int total = wave_incl_scan(nst);
